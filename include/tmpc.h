@@ -72,7 +72,13 @@ typedef struct tmpc_state {
  * n < w the records carry w - n decoupled dummy variables, which never reach
  * the state.  TMPC_FLAG_GENERIC_KERNEL selects the generic per-stage kernel
  * instead (same iteration; for cross-checks).  Bits 8-9 force the number of
- * problems per wavefront of the streaming kernel (1-3; 0 = chosen from B). */
+ * problems per wavefront of the streaming kernel (1-3; 0 = chosen from B).
+ * With TMPC_FLAG_DIAG_COST as well, small blocks (nx <= 13, n - nx <= 4, with
+ * m <= 4 rows, m <= 12 for nx <= 6 and n - nx <= 3, m <= 16 for nx <= 12) and
+ * horizons whose blocks fit a workgroup's LDS and registers run on-chip instead, one
+ * problem per workgroup without stage records, for batches where that is the
+ * faster path; the generic-kernel, bits 8-9 and TMPC_FLAG_FACTOR_GROUPS flags
+ * keep the other kernels. */
 #define TMPC_FLAG_GENERIC_KERNEL 2u
 #define TMPC_FLAG_STREAM_P(p) (((uint32_t)(p) & 3u) << 8)
 /* tmpc_admm_pcg_* with TMPC_FLAG_STD_DYNAMICS runs the whole solve in one
@@ -92,8 +98,8 @@ typedef struct tmpc_state {
 /* Every D_t is diagonal (quadratic costs with per-variable weights), vouched
  * for by the caller.  The streaming kernel then keeps diag(D_t) in its stage
  * records and forms the D_t x terms from it, and the first-order check reads
- * only the diagonal: the same products term by term (ignored by the other
- * paths). */
+ * only the diagonal: the same products term by term.  The on-chip path needs it
+ * (ignored by the other paths). */
 #define TMPC_FLAG_DIAG_COST 4u
 /* Warm stage records (streaming path of tmpc_admm_direct_* and
  * tmpc_sqp_admm_step_*): the workspace holds the stage records of the previous
@@ -101,7 +107,9 @@ typedef struct tmpc_state {
  * that call's only in A_minus and c (an SQP iteration relinearizing explicit
  * dynamics: D, E, q, G, l, u, A0, c0 and the slack weight are unchanged).  Only
  * the A_minus and c records are rewritten.  Vouched for by the caller; the
- * other paths ignore it. */
+ * other paths ignore it: the on-chip path keeps no records and reads the whole
+ * QP, and a streaming call of dims that the on-chip path takes under other
+ * flags packs its records anew. */
 #define TMPC_FLAG_WARM_RECORDS 8u
 /* With TMPC_FLAG_WARM_RECORDS: the QP also differs from the previous call's in
  * G, l and u (inequality rows relinearized at the new iterate, as the obstacle
@@ -128,6 +136,10 @@ typedef struct tmpc_state {
  * products, so the same iterates bit for bit).  Needs no promise from the
  * caller; ignored by the other paths and shapes. */
 #define TMPC_FLAG_INVARIANT_A 64u
+/* TMPC_FLAG_INVARIANT_A is an offer and not a request: the direct solve may run
+ * on the on-chip path, which has no use for it.  A call with that flag alone
+ * keeps the streaming kernel's form. */
+#define TMPC_FLAG_ANY_FORM (1u << 14)
 
 typedef struct tmpc_admm_cfg {
   int32_t max_iter, check_every, adapt_rho_every, pcg_max_iter, use_slack;

@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kWave * kAinvWaves) void ainv_partial_kernel(Dims d
 }
 
 // The OR of the nparts partial masks into the mask words (one workgroup).
-__global__ __launch_bounds__(256) void ainv_reduce_kernel(const uint32_t* __restrict__ part, int nparts,
+static __global__ __launch_bounds__(256) void ainv_reduce_kernel(const uint32_t* __restrict__ part, int nparts,
                                                           uint32_t* __restrict__ mask) {
   __shared__ uint32_t acc[8];
   if (threadIdx.x < 8) acc[threadIdx.x] = 0;

@@ -21,6 +21,7 @@
 #include "adjoint.hpp"
 #include "sqp.hpp"
 #include "merit.hpp"
+#include "resident_api.hpp"
 
 // Workspace of tmpc_admm_direct_noalloc: one copy per GPU, at its own device
 // address, held until the process ends.  Host code never uses this name as an
@@ -558,6 +559,85 @@ StreamArgs<R> stream_args(const AdmmArgs<R>& a, const DirectWs<R>& w, const Dims
   return s;
 }
 
+// The on-chip path's part of the workspace (resident_api.hpp), in place of the
+// stage records: the factor, then the control words and residuals.
+template <typename R>
+struct ResidentWs {
+  R *V, *L, *res;
+  int32_t* ctl;
+};
+
+template <typename R>
+size_t resident_ws_bytes(const Dims& d, int cls) {
+  return align_up(resident_v_bytes(d, sizeof(R), cls)) + align_up(resident_l_bytes(d, sizeof(R), cls)) +
+         align_up((size_t)d.B * 4 * sizeof(int32_t)) + align_up((size_t)d.B * 8 * sizeof(R));
+}
+
+template <typename R>
+ResidentWs<R> carve_resident(void* ws, const Dims& d, int cls) {
+  Carver c{static_cast<char*>(ws)};
+  ResidentWs<R> w;
+  w.V = reinterpret_cast<R*>(c.take<char>(resident_v_bytes(d, sizeof(R), cls)));
+  w.L = reinterpret_cast<R*>(c.take<char>(resident_l_bytes(d, sizeof(R), cls)));
+  w.ctl = c.take<int32_t>((size_t)d.B * 4);
+  w.res = c.take<R>((size_t)d.B * 8);
+  return w;
+}
+
+template <typename R>
+ResArgs<R> resident_args(const AdmmArgs<R>& a, const ResidentWs<R>& w, bool const_g, bool last_chunk,
+                         const tmpc_sqp_step* sq) {
+  ResArgs<R> r;
+  r.d = a.d;
+  r.V = w.V;
+  r.L = w.L;
+  r.D = a.qp.D;
+  r.q = a.qp.q;
+  r.A0 = a.qp.A0;
+  r.Am = a.qp.Am;
+  r.G = a.qp.G;
+  r.l = a.qp.l;
+  r.u = a.qp.u;
+  r.c0 = a.qp.c0;
+  r.c = a.qp.c;
+  r.slack_w = a.qp.slack_w;
+  r.x = a.st.x;
+  r.z = a.st.z;
+  r.y_g = a.st.y_g;
+  r.y_f0 = a.st.y_f0;
+  r.y_f = a.st.y_f;
+  r.xi = a.st.xi;
+  r.rho = a.st.rho;
+  r.ctl = w.ctl;
+  r.res = w.res;
+  r.iters_out = a.iters_out;
+  r.sigma = a.sigma;
+  r.alpha = a.alpha;
+  r.rho_f_factor = a.rho_f_factor;
+  r.eps_abs = a.eps_abs;
+  r.eps_rel = a.eps_rel;
+  r.rho_min = a.rho_min;
+  r.rho_max = a.rho_max;
+  r.rho_tol = a.rho_tol;
+  r.max_iter = a.max_iter;
+  r.check_every = a.check_every;
+  r.adapt_every = a.adapt_every;
+  r.use_slack = a.use_slack;
+  r.it_lo = a.it_lo;
+  r.it_hi = a.it_hi;
+  r.first_chunk = a.first_chunk;
+  r.last_chunk = last_chunk ? 1 : 0;
+  r.const_g = const_g ? 1 : 0;
+  r.chk_conv = sq ? static_cast<R*>(sq->conv) : nullptr;
+  r.chk_eq = sq ? static_cast<R*>(sq->eq_err) : nullptr;
+  r.chk_iq = sq ? static_cast<R*>(sq->ineq_err) : nullptr;
+  r.chk_g = sq ? static_cast<R*>(sq->g_out) : nullptr;
+  r.act_in = sq ? sq->active_in : nullptr;
+  r.act_out = sq ? sq->active_out : nullptr;
+  r.chk_tol = sq ? (R)sq->tol : R(0);
+  return r;
+}
+
 // Iterations after which a rho change (and so a refactorization) can happen:
 // it >= 2, it % adapt_every == 0 and it % check_every == 0 (admm.py:504-508).
 std::vector<int> chunk_bounds(int max_iter, int check_every, int adapt_every) {
@@ -658,7 +738,27 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
   int sp = stream_problems_per_wave(d.B, cfg->flags, stream_wide(dr) && dr.n == 9);
   if (stream_wide(dr) && (cfg->flags & TMPC_FLAG_STREAM_P(3)) == 0)
     sp = std::min(sp, kWave / stream_wide_rows(dr));  // the wide forms' groups are larger
-  const bool stream = std_dyn && (cfg->flags & TMPC_FLAG_GENERIC_KERNEL) == 0 && stream_ok<R>(dr, sp, diag);
+  const bool streamable = std_dyn && stream_ok<R>(dr, sp, diag);
+  // The on-chip path: explicit-integrator structure, diagonal costs, a shape class
+  // whose blocks fit a workgroup, a factor that fits the records' room, and a batch
+  // for which it is the faster one (resident_pays).  A flag that asks for a form of
+  // the streaming or generic kernels keeps those.
+  auto res_plan = [&](bool cg) {
+    const ResPlan p = std_dyn && diag ? resident_plan(d, sizeof(R), cg) : ResPlan{};
+    const bool runs = p.cls >= 0 && resident_ws_bytes<R>(d, p.cls) <= wsb &&
+                      (resident_pays(p.cls, d.B, sizeof(R)) || !streamable);
+    return runs ? p : ResPlan{};
+  };
+  constexpr uint32_t kOtherForm = TMPC_FLAG_GENERIC_KERNEL | TMPC_FLAG_FACTOR_GROUPS | TMPC_FLAG_STREAM_P(3);
+  const bool other_form = (cfg->flags & kOtherForm) != 0 ||
+                          (cfg->flags & (TMPC_FLAG_INVARIANT_A | TMPC_FLAG_ANY_FORM)) == TMPC_FLAG_INVARIANT_A;
+  const ResPlan rp = other_form ? ResPlan{} : res_plan(const_g);
+  const bool resident = rp.cls >= 0;
+  const bool stream = !resident && streamable && (cfg->flags & TMPC_FLAG_GENERIC_KERNEL) == 0;
+  // Warm stage records: the previous call on the workspace left them, unless these
+  // dims run on-chip under other flags (the plan with one G takes the least LDS):
+  // that path keeps no records, so they are packed anew.
+  const bool warm = (cfg->flags & TMPC_FLAG_WARM_RECORDS) != 0 && res_plan(true).cls < 0;
   // the AINV form: asked for, with the resident G rows, at most two problems
   // per wavefront, and the whole workspace
   const bool ainv = stream && const_g && (cfg->flags & TMPC_FLAG_INVARIANT_A) != 0 && ainv_shape_ok(dr, sizeof(R)) && sp <= 2 &&
@@ -667,7 +767,7 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
   QPDev<R> qr = a.qp;  // the QP as the record kernels read it
   if (pad) qr.A0 = w.a0p;
   // warm stage records that a model's own linearization writes directly
-  const bool rows_in_records = stream && (cfg->flags & TMPC_FLAG_WARM_RECORDS) != 0 && !pad;
+  const bool rows_in_records = stream && warm && !pad;
   bool dyn_in_records = false, ineq_in_records = false;
   if (ql) {
     if (d.n != 17 || d.nx != 13) return TMPC_EBADSHAPE;
@@ -711,7 +811,7 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
     st = launch_status();
     if (st) return st;
     if (!stream) a.act = sq->active_out;
-  } else if (sq && !stream) {
+  } else if (sq && !stream && !resident) {
     // generic path: the check kernel on the input iterate, then the activity
     // test, which the ADMM kernel reads as its per-problem start state
     const bool slack = cfg->use_slack && d.m > 0;
@@ -726,7 +826,7 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
     if (st) return st;
     a.act = sq->active_out;
   }
-  if (stream && (cfg->flags & TMPC_FLAG_WARM_RECORDS)) {
+  if (stream && warm) {
     const unsigned gx = (unsigned)((d.B + kRepackProblems - 1) / kRepackProblems);
     // the A_minus and c rows are rewritten unless they did not change or the
     // quadrotor step already wrote them; G, l and u when they changed, unless
@@ -774,8 +874,14 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
     if (st) return st;
     if (hipEventRecord(side->join, side->q) != hipSuccess) return TMPC_ELAUNCH;
   }
-  st = stream ? launch_factor_std<R>(s, dr, w, qr, a.st.rho, a.sigma, a.rho_f_factor, nullptr, fp, diag, fgroups)
-              : launch_factor_qp<R>(s, d, a.qp, a.st.rho, a.sigma, a.rho_f_factor, nullptr, w.thinv);
+  const ResidentWs<R> rw = resident ? carve_resident<R>(ws, d, rp.cls) : ResidentWs<R>{};
+  auto factor_resident = [&](int32_t* ctl) {
+    const ResFactorArgs<R> f{d, a.qp.D, a.qp.Am, a.qp.G, a.qp.A0, a.st.rho, a.sigma, a.rho_f_factor, ctl, rw.V, rw.L};
+    return resident_factor<R>(s, rp.cls, const_g, f) == hipSuccess ? TMPC_OK : TMPC_ELAUNCH;
+  };
+  st = resident ? factor_resident(nullptr)
+       : stream ? launch_factor_std<R>(s, dr, w, qr, a.st.rho, a.sigma, a.rho_f_factor, nullptr, fp, diag, fgroups)
+                : launch_factor_qp<R>(s, d, a.qp, a.st.rho, a.sigma, a.rho_f_factor, nullptr, w.thinv);
   if (side && hipStreamWaitEvent(s, side->join, 0) != hipSuccess) return TMPC_ELAUNCH;
   if (st) return st;
   if (ainv && !side) {
@@ -786,14 +892,18 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
   if (g_iter_events[0] && hipEventRecord(g_iter_events[0], s) != hipSuccess) return TMPC_ELAUNCH;
   for (size_t c = 0; c + 1 < bounds.size(); ++c) {
     if (c > 0) {
-      st = stream ? launch_factor_std<R>(s, dr, w, qr, a.st.rho, a.sigma, a.rho_f_factor, w.ctl, fp, diag, fgroups)
-                  : launch_factor_qp<R>(s, d, a.qp, a.st.rho, a.sigma, a.rho_f_factor, w.ctl, w.thinv);
+      st = resident ? factor_resident(rw.ctl)
+           : stream ? launch_factor_std<R>(s, dr, w, qr, a.st.rho, a.sigma, a.rho_f_factor, w.ctl, fp, diag, fgroups)
+                    : launch_factor_qp<R>(s, d, a.qp, a.st.rho, a.sigma, a.rho_f_factor, w.ctl, w.thinv);
       if (st) return st;
     }
     a.it_lo = bounds[c];
     a.it_hi = bounds[c + 1];
     a.first_chunk = c == 0 ? 1 : 0;
-    if (stream)
+    if (resident) {
+      const ResArgs<R> r = resident_args<R>(a, rw, const_g, c + 2 == bounds.size(), sq);
+      if (resident_iterate<R>(s, rp, r) != hipSuccess) return TMPC_ELAUNCH;
+    } else if (stream)
       launch_stream<R>(s, stream_args<R>(a, w, dr, qr.A0, diag, sq), sp, const_g, ainv);
     else if (std_dyn)
       launch_chunk<R, true>(s, a);
@@ -803,6 +913,7 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
     if (st) return st;
   }
   if (g_iter_events[1] && hipEventRecord(g_iter_events[1], s) != hipSuccess) return TMPC_ELAUNCH;
+  if (resident) return TMPC_OK;  // it writes the state and the non-finite flags itself
   if (stream) {  // the unpack also sets the non-finite flags
     hipLaunchKernelGGL((stage_unpack_kernel<R>),
                        dim3((unsigned)((d.B + kUnpackProblems - 1) / kUnpackProblems), (unsigned)d.T), dim3(256), 0,

@@ -132,9 +132,12 @@ class ADMMSolver:
         if const_g:  # the caller vouches that G_t is the same for every stage and problem
             self._kernel_flags |= _lib.FLAG_CONST_G
         # the stage-invariant A_minus entries stay resident (found on the
-        # device; exact, so on by default wherever the G rows are resident)
+        # device; exact, so on by default wherever the G rows are resident, for
+        # a solve that the on-chip path leaves to the streaming kernel)
         if const_g if invariant_a is None else invariant_a:
             self._kernel_flags |= _lib.FLAG_INVARIANT_A
+        if invariant_a is None:
+            self._kernel_flags |= _lib.FLAG_ANY_FORM
 
     # properties of the reference solver
     schur_solver = property(lambda self: self._schur_solver)
