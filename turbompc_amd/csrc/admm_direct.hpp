@@ -469,8 +469,12 @@ __global__ __launch_bounds__(kWave) void admm_chunk_kernel(AdmmArgs<R> a) {
   }
 }
 
-// Schur-only exact solve S x = rhs from the factor of S (phi read from S).
-template <typename R, int NC>
+// Schur-only exact solve S x = rhs from the factor of S (phi read from S).  The chain
+// over the stages bounds it: with PF (NC > 0) the rows of the next stage's blocks and
+// its vector entry are in flight while a stage is solved. 
+// T = 51, fp64, without / with PF: n = 16, 512 problems 111 / 70 us, 4096 (1024
+// wavefronts, where the reads bound it) 259 / 283; n = 17, 512 problems 136 / 72.
+template <typename R, int NC, bool PF = false>
 __global__ __launch_bounds__(kWave) void blktri_solve_kernel(Dims d, int g, int P, const R* __restrict__ S,
                                                              const R* __restrict__ thinv,
                                                              const R* __restrict__ rhs, R* __restrict__ x) {
@@ -481,43 +485,118 @@ __global__ __launch_bounds__(kWave) void blktri_solve_kernel(Dims d, int g, int 
   const int b = G.prob, i = G.lane, base = G.gid * g;
   R* sw = sv[0] + base;
   R* sr = sv[1] + base;
-  for (int t = 0; t < T; ++t) {
-    R r = (i < n) ? rhs[((size_t)b * T + t) * n + i] : R(0);
-    if (t > 0 && i < n) {
-      // phi_{t-1} w_{t-1}: phi_{t-1} is the sub-diagonal block of block row t
-      const R* row = S + (((size_t)b * T + t) * n + i) * w3;
-      R s = R(0);
-      for (int k = 0; k < n; ++k) s += row[k] * sw[k];
-      r -= s;
-    }
-    if (i < n) sr[i] = r;
-    wsync();
-    if (i < n) {
-      const R wv = sym_row_dot<R, NC>(thinv + ((size_t)t * B + b) * pk, i, n, sr);
-      if (G.live) x[((size_t)b * T + t) * n + i] = wv;
-      sw[i] = wv;
-    }
-    wsync();
-  }
-  R xn = R(0);
-  for (int t = T - 1; t >= 0; --t) {
-    R xt = (i < n) ? x[((size_t)b * T + t) * n + i] : R(0);
-    if (t < T - 1) {
-      if (i < n) sw[i] = xn;
+  if constexpr (PF) {
+    const int ic = min(i, n - 1), ri = (ic * (ic + 1)) >> 1;
+    const bool on = i < n;
+    auto th_row = [&](int t, R (&h)[NC]) {
+      const R* Th = thinv + ((size_t)t * B + b) * pk;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) h[k] = Th[k <= ic ? ri + k : ((k * (k + 1)) >> 1) + ic];
+    };
+    auto dot = [&](const R (&w)[NC], const R* v) {
+      R acc = R(0);
+#pragma unroll
+      for (int k = 0; k < NC; ++k) acc += w[k] * v[k];
+      return acc;
+    };
+    // row ic of phi_{t-1} (t > 0) and of Theta_t^{-1}, rhs_t
+    R f[NC], h[NC], rn;
+    auto fetch = [&](int t) {
+      const R* row = S + (((size_t)b * T + t) * n + ic) * w3;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) f[k] = t > 0 ? row[k] : R(0);
+      th_row(t, h);
+      rn = rhs[((size_t)b * T + t) * n + ic];
+    };
+    fetch(0);
+    if (on) sw[i] = R(0);
+    R wv = R(0);
+    for (int t = 0; t < T; ++t) {
+      R fc[NC], hc[NC];
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        fc[k] = f[k];
+        hc[k] = h[k];
+      }
+      R r = rn;
+      if (t + 1 < T) fetch(t + 1);
       wsync();
-      R s = R(0);
+      r -= dot(fc, sw);
+      if (on) sr[i] = r;
+      wsync();
+      wv = dot(hc, sr);
+      if (on) {
+        if (G.live) x[((size_t)b * T + t) * n + i] = wv;
+        sw[i] = wv;
+      }
+    }
+    // x_{T-1} = w_{T-1}; then column ic of phi_t and row ic of Theta_t^{-1}, w_t
+    auto back = [&](int t) {
+      const R* Sn = S + ((size_t)b * T + t + 1) * n * w3 + ic;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) f[k] = Sn[k * w3];
+      th_row(t, h);
+      rn = x[((size_t)b * T + t) * n + ic];
+    };
+    back(T - 2);  // (T >= 2)
+    for (int t = T - 2; t >= 0; --t) {
+      R fc[NC], hc[NC];
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        fc[k] = f[k];
+        hc[k] = h[k];
+      }
+      const R wt = rn;
+      if (t > 0) back(t - 1);
+      wsync();
+      const R s = dot(fc, sw);  // phi_t^T x_{t+1}
+      if (on) sr[i] = s;
+      wsync();
+      const R xt = wt - dot(hc, sr);
+      if (on) {
+        if (G.live) x[((size_t)b * T + t) * n + i] = xt;
+        sw[i] = xt;
+      }
+    }
+  } else {
+    for (int t = 0; t < T; ++t) {
+      R r = (i < n) ? rhs[((size_t)b * T + t) * n + i] : R(0);
+      if (t > 0 && i < n) {
+        // phi_{t-1} w_{t-1}: phi_{t-1} is the sub-diagonal block of block row t
+        const R* row = S + (((size_t)b * T + t) * n + i) * w3;
+        R s = R(0);
+        for (int k = 0; k < n; ++k) s += row[k] * sw[k];
+        r -= s;
+      }
+      if (i < n) sr[i] = r;
+      wsync();
       if (i < n) {
-        // phi_t^T xt_{t+1}: phi_t = sub-diagonal block of block row t+1
-        const R* Sn = S + ((size_t)b * T + t + 1) * n * w3;
-        for (int k = 0; k < n; ++k) s += Sn[k * w3 + i] * sw[k];
-        sr[i] = s;
+        const R wv = sym_row_dot<R, NC>(thinv + ((size_t)t * B + b) * pk, i, n, sr);
+        if (G.live) x[((size_t)b * T + t) * n + i] = wv;
+        sw[i] = wv;
       }
       wsync();
-      if (i < n) xt -= sym_row_dot<R, NC>(thinv + ((size_t)t * B + b) * pk, i, n, sr);
-      wsync();
     }
-    if (i < n && G.live) x[((size_t)b * T + t) * n + i] = xt;
-    xn = xt;
+    R xn = R(0);
+    for (int t = T - 1; t >= 0; --t) {
+      R xt = (i < n) ? x[((size_t)b * T + t) * n + i] : R(0);
+      if (t < T - 1) {
+        if (i < n) sw[i] = xn;
+        wsync();
+        R s = R(0);
+        if (i < n) {
+          // phi_t^T xt_{t+1}: phi_t = sub-diagonal block of block row t+1
+          const R* Sn = S + ((size_t)b * T + t + 1) * n * w3;
+          for (int k = 0; k < n; ++k) s += Sn[k * w3 + i] * sw[k];
+          sr[i] = s;
+        }
+        wsync();
+        if (i < n) xt -= sym_row_dot<R, NC>(thinv + ((size_t)t * B + b) * pk, i, n, sr);
+        wsync();
+      }
+      if (i < n && G.live) x[((size_t)b * T + t) * n + i] = xt;
+      xn = xt;
+    }
   }
 }
 

@@ -285,13 +285,26 @@ int launch_nonfinite_flags(hipStream_t s, const Dims& d, const StateDev<R>& st, 
   return launch_status();
 }
 
+// factor_kernel in the smallest form that holds n (kc: factor.hpp)
+template <typename R, int SRC>
+void launch_factor(hipStream_t s, const Dims& d, int kc, const QPDev<R>& q, const R* S, const R* rho, R sigma,
+                   R rho_f_factor, int32_t* ctl, R* thinv) {
+  const size_t smem = factor_smem_bytes(d);
+  auto go = [&](auto kernel, int threads) {
+    lds_optin(kernel, smem);
+    hipLaunchKernelGGL(kernel, dim3(d.B), dim3(threads), smem, s, d, kc, q, S, rho, sigma, rho_f_factor, ctl, thinv);
+  };
+  if (d.n <= 8) go(factor_kernel<R, SRC, 8, 1>, 64);
+  else if (d.n <= 16) go(factor_kernel<R, SRC, 8, 2>, 64);
+  else if (d.n <= 32) go(factor_kernel<R, SRC, 16, 2>, 256);
+  else if (d.n <= 48) go(factor_kernel<R, SRC, 16, 3>, 256);
+  else go(factor_kernel<R, SRC, 16, 4>, 256);
+}
+
 template <typename R>
 int launch_factor_qp(hipStream_t s, const Dims& d, const QPDev<R>& q, const R* rho, R sigma,
                      R rho_f_factor, int32_t* ctl, R* thinv) {
-  const size_t smem = factor_smem_bytes(d);
-  lds_optin(factor_kernel<R, SRC_QP>, smem);
-  hipLaunchKernelGGL((factor_kernel<R, SRC_QP>), dim3(d.B), dim3(kWave), smem, s, d, q,
-                     (const R*)nullptr, rho, sigma, rho_f_factor, ctl, thinv);
+  launch_factor<R, SRC_QP>(s, d, d.n, q, nullptr, rho, sigma, rho_f_factor, ctl, thinv);
   return launch_status();
 }
 
@@ -974,19 +987,23 @@ int blktri_factor_impl(hipStream_t s, int B, int T, int n, const R* S, void* ws,
   if (!S) return TMPC_EBADARG;
   const Dims d = to_dims(&td);
   if (!ws || wsb < align_up((size_t)T * B * th_pitch(n) * sizeof(R))) return TMPC_EWORKSPACE;
-  QPDev<R> q{};
-  const size_t smem = factor_smem_bytes(d);
-  lds_optin(factor_kernel<R, SRC_S>, smem);
-  hipLaunchKernelGGL((factor_kernel<R, SRC_S>), dim3(B), dim3(kWave), smem, s, d, q, S,
-                     (const R*)nullptr, R(0), R(0), (int32_t*)nullptr, static_cast<R*>(ws));
+  launch_factor<R, SRC_S>(s, d, n, QPDev<R>{}, S, nullptr, R(0), R(0), nullptr, static_cast<R*>(ws));
   return launch_status();
 }
 
 template <typename R, int NC>
 void launch_blktri_solve_nc(hipStream_t s, const Dims& d, int g, int P, const R* S, const R* th,
                             const R* rhs, R* x) {
-  hipLaunchKernelGGL((blktri_solve_kernel<R, NC>), dim3((d.B + P - 1) / P), dim3(kWave), 0, s, d, g,
-                     P, S, th, rhs, x);
+  const unsigned grid = (unsigned)((d.B + P - 1) / P);
+  if constexpr (NC > 0) {
+    // the prefetching form gains while the chain bounds the solve (4 to 15% at 512 to
+    // 585 wavefronts), is even at 820 and loses 9% at 1024, bound by its reads
+    if (grid <= 640) {
+      hipLaunchKernelGGL((blktri_solve_kernel<R, NC, true>), dim3(grid), dim3(kWave), 0, s, d, g, P, S, th, rhs, x);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((blktri_solve_kernel<R, NC>), dim3(grid), dim3(kWave), 0, s, d, g, P, S, th, rhs, x);
 }
 
 template <typename R>
@@ -1036,11 +1053,14 @@ size_t adjoint_ws_bytes(const Dims& d) {
 // and nb <= 32, reading the QP blocks directly: block capacities NC (Z) and
 // NBC (rows per problem), P problems per wavefront.  Shapes they do not cover take the assembled-matrix path
 // (kkt_assemble_kernel, factor_kernel, blktri_solve_kernel).
-// 0: not covered; 1, 2, 3: the (NC, NBC) capacities (9, 18), (9, 32), (16, 32)
+// 0: not covered; 1, 2, 3: the (NC, NBC) capacities (9, 18), (9, 32), (16, 32); 4: (17, 34),
+// the solve and the residual only (its factorization is factor_kernel's, whose stage is
+// spread over more lanes than rows)
 inline int kkt_rows_form(const KktDims& k) {
   if (k.n <= 9 && k.nb <= 18) return 1;
   if (k.n <= 9 && k.nb <= 32) return 2;
   if (k.n <= 16 && k.nb <= 32) return 3;
+  if (k.n <= 17 && k.nb <= 34) return 4;
   return 0;
 }
 // Problems per wavefront: enough that the launch holds about one wavefront per
@@ -1048,7 +1068,7 @@ inline int kkt_rows_form(const KktDims& k) {
 // and packing beats a second resident wavefront for the sweeps as well: 374 vs
 // 489 us per solve at B = 2048), up to the groups a wavefront holds.
 inline int kkt_rows_p(const KktDims& k) {
-  const int pmax = kkt_rows_form(k) == 1 ? 3 : 2;  // 64 / NBC groups
+  const int form = kkt_rows_form(k), pmax = form == 1 ? 3 : (form == 4 ? 1 : 2);  // 64 / NBC groups
   return std::max(1, std::min(pmax, (k.B + 1023) / 1024));
 }
 inline unsigned kkt_rows_grid(const KktDims& k, int P) { return (unsigned)((k.B + P - 1) / P); }
@@ -1062,10 +1082,13 @@ inline unsigned kkt_rows_grid(const KktDims& k, int P) { return (unsigned)((k.B 
         break;                                                                                                \
       }                                                                                                       \
     }                                                                                                         \
-    if (P >= 2)                                                                                               \
-      hipLaunchKernelGGL((KERNEL<R, NC, NBC, 2>), dim3(kkt_rows_grid(k, 2)), dim3(kWave), 0, s, k, __VA_ARGS__);   \
-    else                                                                                                      \
-      hipLaunchKernelGGL((KERNEL<R, NC, NBC, 1>), dim3(k.B), dim3(kWave), 0, s, k, __VA_ARGS__);                   \
+    if constexpr (2 * NBC <= kWave) {                                                                         \
+      if (P >= 2) {                                                                                           \
+        hipLaunchKernelGGL((KERNEL<R, NC, NBC, 2>), dim3(kkt_rows_grid(k, 2)), dim3(kWave), 0, s, k, __VA_ARGS__); \
+        break;                                                                                                \
+      }                                                                                                       \
+    }                                                                                                         \
+    hipLaunchKernelGGL((KERNEL<R, NC, NBC, 1>), dim3(k.B), dim3(kWave), 0, s, k, __VA_ARGS__);                     \
   } while (0)
 
 template <typename R, int NC, int NBC>
@@ -1104,6 +1127,8 @@ void launch_kkt_rows(hipStream_t s, const KktDims& k, int which, const QPDev<R>&
     case 12: launch_kkt_rows_nc<R, 16, 32>(s, k, P, q, shift, th); break;
     case 13: launch_kkt_solve_nc<R, 16, 32>(s, k, P, q, th, in, out); break;
     case 14: launch_kkt_residual_nc<R, 16, 32>(s, k, q, in, out); break;
+    case 17: launch_kkt_solve_nc<R, 17, 34>(s, k, P, q, th, in, out); break;
+    case 18: launch_kkt_residual_nc<R, 17, 34>(s, k, q, in, out); break;
     default: break;
   }
 }
@@ -1140,18 +1165,19 @@ int adjoint_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp, R* dz,
   // SRC_S) and blktri_solve_kernel.  TMPC_FLAG_GENERIC_KERNEL selects the
   // latter (cross-checks).
   const bool rows = (flags & TMPC_FLAG_GENERIC_KERNEL) == 0 && kkt_rows_form(k) != 0;
+  const bool rows_factor = rows && kkt_rows_form(k) != 4;
   Dims kd{d.B, d.T, d.N, k.nb, 1, 1, 0, k.nb};
-  if (rows) {
+  if (rows_factor) {
     launch_kkt_rows<R>(s, k, 0, q, shift, th, nullptr, nullptr);
-    launch_kkt_rows<R>(s, k, 1, q, nullptr, th, nullptr, x);
   } else {
     hipLaunchKernelGGL((kkt_assemble_kernel<R>), dim3(d.B * d.T), dim3(256), 0, s, k, q, shift, K, dreg, rhs);
-    const size_t smem = factor_smem_bytes(kd);
-    lds_optin(factor_kernel<R, SRC_S>, smem);
-    hipLaunchKernelGGL((factor_kernel<R, SRC_S>), dim3(d.B), dim3(kWave), smem, s, kd, QPDev<R>{}, (const R*)K,
-                       (const R*)nullptr, R(0), R(0), (int32_t*)nullptr, th);
-    launch_blktri_solve_nc<R, 0>(s, kd, k.nb, kWave / k.nb, K, th, rhs, x);
+    // (the coupling blocks' nonzeros: the z columns)
+    launch_factor<R, SRC_S>(s, kd, d.n, QPDev<R>{}, K, nullptr, R(0), R(0), nullptr, th);
   }
+  if (rows)
+    launch_kkt_rows<R>(s, k, 1, q, nullptr, th, nullptr, x);
+  else
+    launch_blktri_solve_nc<R, 0>(s, kd, k.nb, kWave / k.nb, K, th, rhs, x);
   int st = launch_status();
   if (st) return st;
   for (int it = 0; it < steps; ++it) {
@@ -1197,7 +1223,7 @@ PcgVecs<R> carve_vecs(Carver& c, const Dims& d, R* x) {
 template <typename R>
 int launch_schur_build(hipStream_t s, const Dims& d, const QPDev<R>& q, const R* rho, R sigma, R rfac,
                        int32_t* ctl, R* S, R* Phi) {
-  const size_t smem = factor_smem_bytes(d);
+  const size_t smem = schur_build_smem_bytes(d);
   lds_optin(schur_build_kernel<R>, smem);
   hipLaunchKernelGGL((schur_build_kernel<R>), dim3(d.B), dim3(kWave), smem, s, d, q, rho, sigma, rfac, ctl,
                      S, Phi);

@@ -337,6 +337,17 @@ __global__ __launch_bounds__(64) void nonfinite_flag_kernel(Dims d, StateDev<R> 
 // ordered by this barrier (a single-wave s_barrier is cheap on CDNA).
 __device__ __forceinline__ void wsync() { __syncthreads(); }
 
+// 1/d by the hardware reciprocal estimate refined with two Newton-Raphson
+// steps r <- r + r (1 - d r) (each roughly squares the relative error; d is
+// a pivot of an SPD or quasi-definite block, far from the denormal and overflow ranges)
+__device__ __forceinline__ double recip(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  double e = __builtin_fma(-d, r, 1.0);
+  r = __builtin_fma(r, e, r);
+  e = __builtin_fma(-d, r, 1.0);
+  return __builtin_fma(r, e, r);
+}
+
 // Orders LDS accesses between lanes of one wavefront without waiting: the LDS
 // unit executes one wavefront's instructions in issue order, so a read issued
 // after another lane's write returns the written value; only the compiler has

@@ -222,17 +222,6 @@ __device__ __forceinline__ double fac_dot(const double (&w)[N], double s) {
   return row_dot_dpp(v, s);
 }
 
-// 1/d by the hardware reciprocal estimate refined with two Newton-Raphson
-// steps r <- r + r (1 - d r) (each roughly squares the relative error; d is
-// a pivot of an SPD block, far from the denormal and overflow ranges)
-__device__ __forceinline__ double recip(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  double e = __builtin_fma(-d, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-d, r, 1.0);
-  return __builtin_fma(r, e, r);
-}
-
 template <int KP, int NL, typename F>
 __device__ __forceinline__ void static_for_pivots(F&& f) {
   if constexpr (KP < NL) {

@@ -22,6 +22,39 @@
 namespace tmpc {
 
 // ------------------------------------------------------------ S / Phiinv ----
+template <typename C>
+__device__ void gj_invert_spd(C* A, C* rowk, C* colk, int n) {
+  const int tid = threadIdx.x;
+  const int nn = n * n;
+  for (int k = 0; k < n; ++k) {
+    if (tid < n) {
+      rowk[tid] = A[k * n + tid];
+      colk[tid] = A[tid * n + k];
+    }
+    wsync();
+    const C ip = C(1) / rowk[k];
+    for (int e = tid; e < nn; e += kWave) {
+      const int i = e / n, j = e - (e / n) * n;
+      C v;
+      if (i == k && j == k)
+        v = ip;
+      else if (i == k)
+        v = rowk[j] * ip;
+      else if (j == k)
+        v = -colk[i] * ip;
+      else
+        v = A[e] - colk[i] * rowk[j] * ip;
+      A[e] = v;
+    }
+    wsync();
+  }
+}
+
+inline size_t schur_build_smem_bytes(const Dims& d) {
+  const size_t n = d.n;
+  return sizeof(Cmp) * (4 * n * n + 2 * n + (size_t)d.m * n + 3 * (size_t)d.nx * n + (size_t)d.n0 * n);
+}
+
 template <typename R>
 __global__ __launch_bounds__(kWave) void schur_build_kernel(Dims d, QPDev<R> qp, const R* __restrict__ rho,
                                                             R sigma, R rho_f_factor,
