@@ -22,15 +22,17 @@ constexpr size_t kLdsBytes = 160 * 1024;
 // so the time grows with B from 256 on; the streaming kernel leaves the chip idle up
 // to about 2048 problems and then runs at its rate over memory.  QP solves of 20
 // iterations, on-chip / streaming in us:
-//   C4 fp32, T = 41: 334 / 1404 at B = 256, 1072 / 1688 at 2048, 1594 / 1924 at 3072,
-//     2047 / 2109 at 4096 (there the streaming kernel's records, which an SQP step
-//     relinearizes in place, decide); T = 21: 644 / 910 at 2048, 1230 / 1151 at 4096
-//   C4 fp64, T = 41: 409 / 1626 at 256, 2115 / 2176 at 2048, 4202 / 4176 at 4096
-//   C1 fp32, T = 101: 995 / 5292 at 512, 3541 / 5490 at 2048, 6927 / 6785 at 4096;
-//     fp64: 1177 / 6247 at 512, 4255 / 6669 at 2048, 8386 / 14622 at 4096
-//   C2 fp32, T = 61: 1418 / 2663 at 2048, 10162 / 12974 at 16384; fp64, T = 48:
-//     2535 / 2653 at 2048, 4877 / 5102 at 4096
-//   C3, T = 51: 680 / 2763 at 512, 4277 / 10608 at 4096; fp64 910 / 3372 at 512
+//   C4 fp32, T = 41: 319 / 1412 at B = 256, 1029 / 1696 at 2048, 1534 / 1909 at 3072,
+//     1951 / 2081 at 4096 (there the streaming kernel's records, which an SQP step
+//     relinearizes in place, decide: 5 steps 10222 / 10038); T = 21: 626 / 912 at 2048,
+//     1179 / 1110 at 4096
+//   C4 fp64, T = 41: 399 / 1629 at 256, 2053 / 2171 at 2048, 4060 / 4171 at 4096
+//   C1 fp32, T = 101: 925 / 5285 at 512, 3275 / 5495 at 2048, 6772 / 6778 at 4096 (50
+//     iterations; 2840 / 3181 of 20); fp64: 1175 / 6259 at 512, 4267 / 6663 at 2048,
+//     8384 / 14317 at 4096
+//   C2 fp32, T = 61: 1385 / 2675 at 2048, 9950 / 12842 at 16384; fp64, T = 48:
+//     2542 / 2657 at 2048, 4901 / 5118 at 4096
+//   C3, T = 51: 660 / 2758 at 512, 4060 / 10603 at 4096; fp64 908 / 3353 at 512
 //   C0 fp64, T = 21: 169 / 778 at 64, 944 / 964 at 4096, 3598 / 3572 at 16384; fp32:
 //     556 / 836 at 4096, 1761 / 2460 at 16384
 template <int NX_, int NU_, int MM_, int GL_, int KF_, int KD_, int K64_, int BF_, int B64_>
@@ -38,10 +40,10 @@ struct Cls {
   static constexpr int NX = NX_, NU = NU_, MM = MM_, GL = GL_, KF = KF_, KD = KD_, K64 = K64_, BF = BF_, B64 = B64_;
 };
 using C0 = Cls<4, 2, 4, 16, 4, 0, 4, 0, 16>;
-using C1 = Cls<6, 3, 4, 16, 4, 0, 7, 12, 0>;
+using C1 = Cls<6, 3, 4, 16, 4, 0, 7, 16, 0>;
 using C2 = Cls<6, 3, 12, 32, 4, 8, 8, 0, 0>;
 using C3 = Cls<12, 4, 16, 32, 4, 0, 7, 0, 0>;
-using C4 = Cls<13, 4, 4, 32, 4, 6, 6, 12, 8>;
+using C4 = Cls<13, 4, 4, 32, 4, 6, 6, 12, 16>;
 constexpr int kClasses = 5;
 
 template <typename F>

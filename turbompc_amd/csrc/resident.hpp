@@ -17,11 +17,11 @@
 //   P2  u_t = Suu^-1 (gu_t + rho_f A_u^T x_{t+1}) - Kx x_t, products, relaxation,
 //       projection, duals, gamma_t -> gx_t = gamma_x - Kx^T gu, h_t  (all stages)
 // with a workgroup barrier after each.  Cycles of an iteration (C1, P1, C2, P2, waits
-// and the rest): fp32, T = 41, NX = 13, alone on its CU 4780 + 1150 + 4160 + 4340 +
-// 3150, two workgroups on each 5070 + 2200 + 4400 + 9360 + 3050; fp64, T = 101,
+// and the rest): fp32, T = 41, NX = 13, alone on its CU 3380 + 1140 + 3750 + 4360 +
+// 3150, two workgroups on each 4340 + 2000 + 4120 + 9170 + 3130; fp64, T = 101,
 // NX = 6 5730 + 1770 + 7330 + 7480 + 1940.  QP solves of 20 iterations against the
 // streaming kernel, which reads every record twice per iteration and walks all T
-// stages in turn, are listed at the shape classes (resident.hip): 1404 -> 334 us for
+// stages in turn, are listed at the shape classes (resident.hip): 1412 -> 319 us for
 // 256 problems of T = 41, NX = 13 in fp32.
 //
 // A stage is a group of GL lanes: GL = 32 has the states (and dynamics rows) in the
@@ -493,10 +493,10 @@ __global__ __launch_bounds__(TPB, WPE) void admm_resident_kernel(ResArgs<R> a) {
   // The chains, in the first 32 lanes: row 0 from position 0 to mid, row 1 from mid + 1
   // to end, mid steps each.  Records are fetched CB - 1 positions ahead, in CB register
   // sets used by turns: an LDS read of a record takes longer than a step of NX <= 6
-  // (fp64, NX = 6: 178 cycles a step with two sets, 141 with three), about as long as a
-  // longer one, for which a third set costs spills (fp32, NX = 13, 4096 problems: 2173 us
-  // with two sets, 2496 with three).
-  constexpr int CB = NX <= 6 ? 3 : 2;
+  // (fp64, NX = 6: 178 cycles a step with two sets, 141 with three; fp32, NX = 12: 190 and
+  // 158); where wide blocks and many stages per group fill the registers, a third set
+  // costs spills (fp32, NX = 13, 4096 problems: 2173 us with two sets, 2496 with three).
+  constexpr int CB = (NX <= 6 || TPB == 512) ? 3 : 2;
   const bool bw = (lane & 16) != 0;
   R* const cb = sC + (bw ? (mid + 1) * CW : 0);
   struct CBuf {
@@ -505,13 +505,19 @@ __global__ __launch_bounds__(TPB, WPE) void admm_resident_kernel(ResArgs<R> a) {
   auto ld_row = [&](CBuf& c, const R* q) __attribute__((always_inline)) {  // gx, h and V's row
     c.g = q[Rec::gx + lc];
     c.h = q[Rec::h + lc];
-    const V16* p = reinterpret_cast<const V16*>(q + lc * W);
+    const R* p = q + lc * W;
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
-      const V16 v = p[k * NX];
+      if (k * W + W <= NX) {
+        const V16 v = *reinterpret_cast<const V16*>(p + k * NX * W);
 #pragma unroll
-      for (int e = 0; e < W; ++e)
-        if (k * W + e < NX) c.w[k * W + e] = v[e];
+        for (int e = 0; e < W; ++e) c.w[k * W + e] = v[e];
+      } else {  // the last entries alone: the registers of a whole chunk's rest would be
+                // given to other values, which then wait for the load (fp32, NX = 13: 210
+                // cycles a step, 170 like this)
+#pragma unroll
+        for (int e = 0; k * W + e < NX; ++e) c.w[k * W + e] = p[k * NX * W + e];
+      }
     }
   };
   const int vcol = (lc / W) * NX * W + lc % W;
