@@ -160,3 +160,25 @@ def test_resident_leaves_no_warm_records():
         want = out if want is None else want
         for k in FIELDS:
             assert torch.equal(getattr(out, k), getattr(want, k)), (warm, k)
+
+
+@pytest.mark.parametrize("shape", [(5, 17, 13, 4), (6, 9, 6, 11), (4, 16, 12, 9)])
+def test_resident_factor_one_and_two_wavefronts(shape):
+    """The factorization with a wavefront of its own for the preparation (up to 1024
+    problems) and without: the same bits."""
+    T, n, nx, m = shape
+    qp = random_qp(1026, T, n, nx, m, seed=96, std=True, diag=True)
+    part = type(qp)(**{f.name: getattr(qp, f.name) for f in dataclasses.fields(qp)})
+    part = dataclasses.replace(
+        part, **{f.name: dataclasses.replace(getattr(qp, f.name), **{
+            g.name: getattr(getattr(qp, f.name), g.name)[:7] for g in dataclasses.fields(getattr(qp, f.name))
+            if torch.is_tensor(getattr(getattr(qp, f.name), g.name)) and getattr(getattr(qp, f.name), g.name).ndim > 0})
+            for f in dataclasses.fields(qp) if dataclasses.is_dataclass(getattr(qp, f.name))})
+    outs = []
+    for q in (qp, part):
+        st = _state_to_dev(zero_state(q, 0.1), torch.float64)
+        (_, _), _, out = _solver(q, _cfg(), std_dynamics=True, diag_cost=True).solve(q.to(DEV, torch.float64), st)
+        outs.append(out)
+    torch.cuda.synchronize()
+    for k in FIELDS:
+        assert torch.equal(getattr(outs[0], k)[:7], getattr(outs[1], k)), k

@@ -58,6 +58,7 @@ auto with_class(int cls, F&& f) {
 }
 
 constexpr int kCUs = 256;
+constexpr int kSplitProblems = 4 * kCUs;
 
 template <typename R>
 ResPlan plan(const Dims& d, int cls, bool const_g) {
@@ -133,10 +134,25 @@ hipError_t resident_factor(hipStream_t s, int cls, bool const_g, const ResFactor
   with_class(cls, [&](auto c) {
     using C = decltype(c);
     const dim3 grid((unsigned)((a.d.B + 1) / 2));
-    if (const_g)
-      hipLaunchKernelGGL((resident_factor_kernel<R, C::NX, C::NU, C::MM, true>), grid, dim3(kWave), 0, s, a);
-    else
-      hipLaunchKernelGGL((resident_factor_kernel<R, C::NX, C::NU, C::MM, false>), grid, dim3(kWave), 0, s, a);
+    auto launch = [&](auto split) {
+      constexpr bool SP = decltype(split)::value;
+      const dim3 block(SP ? 2 * kWave : kWave);
+      if (const_g)
+        hipLaunchKernelGGL((resident_factor_kernel<R, C::NX, C::NU, C::MM, true, SP>), grid, block, 0, s, a);
+      else
+        hipLaunchKernelGGL((resident_factor_kernel<R, C::NX, C::NU, C::MM, false, SP>), grid, block, 0, s, a);
+    };
+    // Two wavefronts for two problems while that leaves a SIMD to each.  Factorization and
+    // one iteration, one wavefront / two, us: C4 fp32, T = 41 176 / 139 for one problem,
+    // 241 / 208 for 1024, 359 / 395 for 2048; C2, T = 61 230 / 210 for 1024, 530 / 583 for
+    // 4096; C3, T = 51 273 / 236 for 1024, 406 / 436 for 2048; C0 (blocks too small to pay
+    // for the exchange) fp64, T = 21 87.4 / 90.6 for 64.
+    if constexpr (C::NX > 4)
+      if (a.d.B <= kSplitProblems) {
+        launch(std::true_type{});
+        return 0;
+      }
+    launch(std::false_type{});
     return 0;
   });
   return hipGetLastError();

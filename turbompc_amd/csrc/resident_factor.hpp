@@ -14,6 +14,12 @@
 //        Theta_m = X_m minus both sides' terms.
 // fp64 throughout, rounded on store.
 //
+// The steps' serial chain bounds small batches.  With SPLIT a workgroup has two
+// wavefronts: one prepares step s + 1 (what does not follow from other stages: gram,
+// control elimination) while the other eliminates step s; the blocks pass through LDS.
+// One problem of T = 41, NX = 13: 117 -> 80 us; a launch that fills the SIMDs anyway
+// loses (16384 problems of T = 61, NX = 6: 844 -> 1080 us).
+//
 // A wavefront holds two problems, each in two 16-lane rows, one per direction: lane
 // i of a row owns row i of every nx x nx block, and everything that crosses lanes
 // goes by DPP row broadcasts (row_dpp.hpp).  A row's step handles the stage p it
@@ -78,14 +84,16 @@ __device__ __forceinline__ void row_inverse(double (&a)[NX], int i, double (*sym
 }
 
 // CG: G_t is the same for every stage and problem (its gram is formed once)
-template <typename R, int NX, int NU, int MM, bool CG>
-__global__ __launch_bounds__(kWave) void resident_factor_kernel(ResFactorArgs<R> a) {
+template <typename R, int NX, int NU, int MM, bool CG, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 2 * kWave : kWave) void resident_factor_kernel(ResFactorArgs<R> a) {
   using Ge = ResGeom<R, NX, NU>;
   constexpr int W = Ge::W;
   __shared__ double sym_all[4][16][NX + 1];
+  __shared__ double prep[SPLIT ? 2 : 1][3][SPLIT ? NX : 1][kWave];  // own, xn, qq of a step, by turns
   const Dims d = a.d;
   const int T = d.T, N = d.N, n = d.n, nx = d.nx, nu = d.n - d.nx, m = d.m, B = d.B;
-  const int lane = threadIdx.x, q4 = lane >> 4, i = lane & 15;
+  const bool chain = SPLIT && threadIdx.x < kWave;  // wavefront 0 eliminates, wavefront 1 prepares
+  const int lane = threadIdx.x & (kWave - 1), q4 = lane >> 4, i = lane & 15;
   const bool bwd = (q4 & 1) != 0;
   const int b0 = blockIdx.x * 2;
   const int np = min(2, B - b0);
@@ -169,7 +177,7 @@ __global__ __launch_bounds__(kWave) void resident_factor_kernel(ResFactorArgs<R>
 #pragma unroll
     for (int k = 0; k < NU; ++k) gxu[k] = guu[k] = 0.0;
   };
-  if constexpr (CG) {
+  if (CG && !chain) {
     double gc[MM], gu[MM], gr[NU];
 #pragma unroll
     for (int j = 0; j < MM; ++j) {
@@ -193,15 +201,11 @@ __global__ __launch_bounds__(kWave) void resident_factor_kernel(ResFactorArgs<R>
     }
   };
 
-  double part[NX];
-#pragma unroll
-  for (int k = 0; k < NX; ++k) part[k] = 0.0;
-  load(0);
-  for (int s = 0; s <= S; ++s) {
-    const int p = stage_of(s), t = bwd ? p + 1 : p;
-    const bool valid = bwd ? s <= nb : (s >= 1 && s <= nf);
-    const bool step = valid && s >= 1;
-    double col[NX], au[NU], own[NX], xu[NU], uu[NU], qq[NX];
+  auto valid_step = [&](int s) { return bwd ? s <= nb : (s >= 1 && s <= nf); };
+  auto prepare = [&](int s, double (&own)[NX], double (&xn)[NX], double (&qq)[NX]) __attribute__((always_inline)) {
+    const int p = stage_of(s);
+    const bool valid = valid_step(s);
+    double col[NX], au[NU], xu[NU], uu[NU];
 #pragma unroll
     for (int r = 0; r < NX; ++r) col[r] = (double)nx_.col[r];
 #pragma unroll
@@ -306,7 +310,6 @@ __global__ __launch_bounds__(kWave) void resident_factor_kernel(ResFactorArgs<R>
         }
       }
     }
-    double xn[NX];
 #pragma unroll
     for (int k = 0; k < NX; ++k) xn[k] = 0.0;
 #pragma unroll
@@ -315,10 +318,19 @@ __global__ __launch_bounds__(kWave) void resident_factor_kernel(ResFactorArgs<R>
       row_axpy(xn, kn[k], rf * au[k]);
       row_axpy(qq, bwd ? au[k] : kx[k], rf * (bwd ? kx[k] : au[k]));
     }
+  };
+  double part[NX];
+#pragma unroll
+  for (int k = 0; k < NX; ++k) part[k] = 0.0;
+  auto eliminate = [&](int s, const double (&own)[NX], const double (&xn)[NX], const double (&qq)[NX])
+                       __attribute__((always_inline)) {
+    const int p = stage_of(s), t = bwd ? p + 1 : p;
+    const bool valid = valid_step(s);
+    const bool step = valid && s >= 1;
     if (s == 0) {  // only the last stage's own block (towards lower t)
 #pragma unroll
       for (int k = 0; k < NX; ++k) part[k] = valid ? own[k] : part[k];
-      continue;
+      return;
     }
     double th[NX];
 #pragma unroll
@@ -339,6 +351,39 @@ __global__ __launch_bounds__(kWave) void resident_factor_kernel(ResFactorArgs<R>
     for (int k = 0; k < NX; ++k) row_axpy(th, qq[k], y[k]);
 #pragma unroll
     for (int k = 0; k < NX; ++k) part[k] = valid ? (bwd ? own[k] : xn[k]) - th[k] : part[k];
+  };
+  if (!chain) load(0);
+  double own[NX], xn[NX], qq[NX];
+  if constexpr (SPLIT) {
+    for (int s = 0; s <= S + 1; ++s) {  // step s prepared while step s - 1 is eliminated
+      auto& buf = prep[chain ? (s + 1) & 1 : s & 1];
+      if (chain) {
+        if (s >= 1) {
+#pragma unroll
+          for (int k = 0; k < NX; ++k) {
+            own[k] = buf[0][k][lane];
+            xn[k] = buf[1][k][lane];
+            qq[k] = buf[2][k][lane];
+          }
+          eliminate(s - 1, own, xn, qq);
+        }
+      } else if (s <= S) {
+        prepare(s, own, xn, qq);
+#pragma unroll
+        for (int k = 0; k < NX; ++k) {
+          buf[0][k][lane] = own[k];
+          buf[1][k][lane] = xn[k];
+          buf[2][k][lane] = qq[k];
+        }
+      }
+      __syncthreads();
+    }
+    if (!chain) return;
+  } else {
+    for (int s = 0; s <= S; ++s) {
+      prepare(s, own, xn, qq);
+      eliminate(s, own, xn, qq);
+    }
   }
   // the middle stage: both directions' terms
 #pragma unroll
