@@ -470,9 +470,10 @@ def run_config5(args, dev):
                          "parallelism": "single GPU, batch-parallel", "solution_finite": finite,
                          "forward_qp_solve_ms": solve_avg_s * 1e3, "backward_ms": bwd_avg_ms})
     line["roofline"] = roofline(
-        achieved, None, f"admm_stream_kernel, fp64 (one launch = {K} ADMM iterations of the batch)", iter_bytes,
+        achieved, None, f"admm_resident_kernel, fp64 (one launch = {K} ADMM iterations of the batch; the bytes are the "
+        "streaming model's, which this kernel does not move: its blocks stay in LDS and registers)", iter_bytes,
         iter_avg_s * 1e3,
-        qp_solve={"kernels": "stage_pack + factor_row + admm_stream + stage_unpack", "algorithmic_bytes": per_qp * B,
+        qp_solve={"kernels": "resident_factor + admm_resident", "algorithmic_bytes": per_qp * B,
                   "avg_ms": solve_avg_s * 1e3, "achieved": per_qp * B / solve_avg_s / 1e9,
                   "frac": per_qp * B / solve_avg_s / 1e9 / HBM_PEAK_GBS})
     return line
