@@ -253,7 +253,7 @@ __device__ __forceinline__ double row_dot_dpp(const double (&w)[6], double s) {
       "v_fmac_f64_dpp %0, %2, %7 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %8 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]));
   return a0 + a1;
 }
@@ -272,7 +272,7 @@ __device__ __forceinline__ double row_dot_dpp(const double (&w)[9], double s) {
       "v_fmac_f64_dpp %1, %2, %10 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %11 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]));
   return a0 + a1;
 }
@@ -298,7 +298,7 @@ __device__ __forceinline__ double row_dot_dpp(const double (&w)[16], double s) {
       "v_fmac_f64_dpp %0, %2, %17 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %18 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]), "v"(w[13]), "v"(w[14]), "v"(w[15]));
   return a0 + a1;
 }

@@ -51,7 +51,7 @@ __device__ __forceinline__ void axpy_bcast6(double (&c)[N], double src, double s
       "v_fmac_f64_dpp %4, %6, %7 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %5, %6, %7 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5])
+      : "+&v"(c[0]), "+&v"(c[1]), "+&v"(c[2]), "+&v"(c[3]), "+&v"(c[4]), "+&v"(c[5])
       : "v"(src), "v"(s));
 }
 
@@ -70,7 +70,7 @@ __device__ __forceinline__ void axpy_bcast9(double (&c)[N], double src, double s
       "v_fmac_f64_dpp %7, %9, %10 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %8, %9, %10 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5]), "+v"(c[6]), "+v"(c[7]), "+v"(c[8])
+      : "+&v"(c[0]), "+&v"(c[1]), "+&v"(c[2]), "+&v"(c[3]), "+&v"(c[4]), "+&v"(c[5]), "+&v"(c[6]), "+&v"(c[7]), "+&v"(c[8])
       : "v"(src), "v"(s));
 }
 
@@ -96,7 +96,7 @@ __device__ __forceinline__ void axpy_bcast16(double (&c)[N], double src, double 
       "v_fmac_f64_dpp %14, %16, %17 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %15, %16, %17 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5]), "+v"(c[6]), "+v"(c[7]), "+v"(c[8]), "+v"(c[9]), "+v"(c[10]), "+v"(c[11]), "+v"(c[12]), "+v"(c[13]), "+v"(c[14]), "+v"(c[15])
+      : "+&v"(c[0]), "+&v"(c[1]), "+&v"(c[2]), "+&v"(c[3]), "+&v"(c[4]), "+&v"(c[5]), "+&v"(c[6]), "+&v"(c[7]), "+&v"(c[8]), "+&v"(c[9]), "+&v"(c[10]), "+&v"(c[11]), "+&v"(c[12]), "+&v"(c[13]), "+&v"(c[14]), "+&v"(c[15])
       : "v"(src), "v"(s));
 }
 
@@ -114,7 +114,7 @@ __device__ __forceinline__ void sweep_bcast6(double (&a)[N], double g) {
       "v_fmac_f64_dpp %4, %4, %6 row_newbcast:%c7 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %5, %5, %6 row_newbcast:%c7 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5])
+      : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5])
       : "v"(g), "i"(KP));
 }
 
@@ -133,7 +133,7 @@ __device__ __forceinline__ void sweep_bcast9(double (&a)[N], double g) {
       "v_fmac_f64_dpp %7, %7, %9 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %8, %8, %9 row_newbcast:%c10 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8])
+      : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7]), "+&v"(a[8])
       : "v"(g), "i"(KP));
 }
 
@@ -159,7 +159,7 @@ __device__ __forceinline__ void sweep_bcast16(double (&a)[N], double g) {
       "v_fmac_f64_dpp %14, %14, %16 row_newbcast:%c17 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %15, %15, %16 row_newbcast:%c17 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), "+v"(a[12]), "+v"(a[13]), "+v"(a[14]), "+v"(a[15])
+      : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7]), "+&v"(a[8]), "+&v"(a[9]), "+&v"(a[10]), "+&v"(a[11]), "+&v"(a[12]), "+&v"(a[13]), "+&v"(a[14]), "+&v"(a[15])
       : "v"(g), "i"(KP));
 }
 
@@ -186,7 +186,7 @@ __device__ __forceinline__ void sweep_bcast17(double (&a)[N], double g) {
       "v_fmac_f64_dpp %15, %15, %17 row_newbcast:%c18 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %16, %16, %17 row_newbcast:%c18 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), "+v"(a[12]), "+v"(a[13]), "+v"(a[14]), "+v"(a[15]), "+v"(a[16])
+      : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7]), "+&v"(a[8]), "+&v"(a[9]), "+&v"(a[10]), "+&v"(a[11]), "+&v"(a[12]), "+&v"(a[13]), "+&v"(a[14]), "+&v"(a[15]), "+&v"(a[16])
       : "v"(g), "i"(KP));
 }
 

@@ -5,7 +5,9 @@
 // so the blocks are written out.  Each block starts with the wait states a DPP
 // read needs after a VALU write of its source; a result is last written by an
 // ordinary instruction (the final add), or the block ends with wait states.
-// Every lane of the wavefront must be active.
+// Accumulators are early-clobber operands ("+&v"): later instructions of a block
+// still read its sources, also where one holds an accumulator's starting value.
+// Every lane of a 16-lane row that is active at all must be active.
 #pragma once
 #include "common.hpp"
 
@@ -23,7 +25,7 @@ __device__ __forceinline__ float row_fma(const float (&w)[2], float s, float acc
       "s_nop 1\n"
       "v_fmac_f32_dpp %0, %2, %3 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n"
       "v_mul_f32_dpp %1, %2, %4 row_newbcast:%c6 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "=&v"(odd)
+      : "+&v"(acc), "=&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "n"(O + 0), "n"(O + 1));
   return acc + odd;
 }
@@ -37,7 +39,7 @@ __device__ __forceinline__ float row_fma(const float (&w)[3], float s, float acc
       "v_fmac_f32_dpp %0, %2, %3 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n"
       "v_mul_f32_dpp %1, %2, %4 row_newbcast:%c7 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %0, %2, %5 row_newbcast:%c8 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "=&v"(odd)
+      : "+&v"(acc), "=&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "n"(O + 0), "n"(O + 1), "n"(O + 2));
   return acc + odd;
 }
@@ -52,7 +54,7 @@ __device__ __forceinline__ float row_fma(const float (&w)[4], float s, float acc
       "v_mul_f32_dpp %1, %2, %4 row_newbcast:%c8 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %0, %2, %5 row_newbcast:%c9 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %6 row_newbcast:%c10 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "=&v"(odd)
+      : "+&v"(acc), "=&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3));
   return acc + odd;
 }
@@ -69,7 +71,7 @@ __device__ __forceinline__ float row_fma(const float (&w)[6], float s, float acc
       "v_fmac_f32_dpp %1, %2, %6 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %0, %2, %7 row_newbcast:%c13 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %8 row_newbcast:%c14 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "=&v"(odd)
+      : "+&v"(acc), "=&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3), "n"(O + 4), "n"(O + 5));
   return acc + odd;
 }
@@ -92,7 +94,7 @@ __device__ __forceinline__ float row_fma(const float (&w)[12], float s, float ac
       "v_fmac_f32_dpp %1, %2, %12 row_newbcast:%c24 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %0, %2, %13 row_newbcast:%c25 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %14 row_newbcast:%c26 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "=&v"(odd)
+      : "+&v"(acc), "=&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3), "n"(O + 4), "n"(O + 5), "n"(O + 6), "n"(O + 7), "n"(O + 8), "n"(O + 9), "n"(O + 10), "n"(O + 11));
   return acc + odd;
 }
@@ -116,7 +118,7 @@ __device__ __forceinline__ float row_fma(const float (&w)[13], float s, float ac
       "v_fmac_f32_dpp %0, %2, %13 row_newbcast:%c26 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %14 row_newbcast:%c27 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %0, %2, %15 row_newbcast:%c28 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "=&v"(odd)
+      : "+&v"(acc), "=&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3), "n"(O + 4), "n"(O + 5), "n"(O + 6), "n"(O + 7), "n"(O + 8), "n"(O + 9), "n"(O + 10), "n"(O + 11), "n"(O + 12));
   return acc + odd;
 }
@@ -129,7 +131,7 @@ __device__ __forceinline__ double row_fma(const double (&w)[2], double s, double
       "s_nop 1\n"
       "v_fmac_f64_dpp %0, %2, %3 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %4 row_newbcast:%c6 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "n"(O + 0), "n"(O + 1));
   return acc + odd;
 }
@@ -143,7 +145,7 @@ __device__ __forceinline__ double row_fma(const double (&w)[3], double s, double
       "v_fmac_f64_dpp %0, %2, %3 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %4 row_newbcast:%c7 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %5 row_newbcast:%c8 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "n"(O + 0), "n"(O + 1), "n"(O + 2));
   return acc + odd;
 }
@@ -158,7 +160,7 @@ __device__ __forceinline__ double row_fma(const double (&w)[4], double s, double
       "v_fmac_f64_dpp %1, %2, %4 row_newbcast:%c8 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %5 row_newbcast:%c9 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %6 row_newbcast:%c10 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3));
   return acc + odd;
 }
@@ -175,7 +177,7 @@ __device__ __forceinline__ double row_fma(const double (&w)[6], double s, double
       "v_fmac_f64_dpp %1, %2, %6 row_newbcast:%c12 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %7 row_newbcast:%c13 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %8 row_newbcast:%c14 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3), "n"(O + 4), "n"(O + 5));
   return acc + odd;
 }
@@ -198,7 +200,7 @@ __device__ __forceinline__ double row_fma(const double (&w)[12], double s, doubl
       "v_fmac_f64_dpp %1, %2, %12 row_newbcast:%c24 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %13 row_newbcast:%c25 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %14 row_newbcast:%c26 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3), "n"(O + 4), "n"(O + 5), "n"(O + 6), "n"(O + 7), "n"(O + 8), "n"(O + 9), "n"(O + 10), "n"(O + 11));
   return acc + odd;
 }
@@ -222,7 +224,7 @@ __device__ __forceinline__ double row_fma(const double (&w)[13], double s, doubl
       "v_fmac_f64_dpp %0, %2, %13 row_newbcast:%c26 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %14 row_newbcast:%c27 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %15 row_newbcast:%c28 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3), "n"(O + 4), "n"(O + 5), "n"(O + 6), "n"(O + 7), "n"(O + 8), "n"(O + 9), "n"(O + 10), "n"(O + 11), "n"(O + 12));
   return acc + odd;
 }
@@ -236,7 +238,7 @@ __device__ __forceinline__ float row_fma_seed(const float (&w)[4], float s, floa
       "v_fmac_f32_dpp %1, %2, %4 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %0, %2, %5 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %6 row_newbcast:3 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]));
   return acc + odd;
 }
@@ -250,7 +252,7 @@ __device__ __forceinline__ float row_fma_seed(const float (&w)[6], float s, floa
       "v_fmac_f32_dpp %1, %2, %6 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %0, %2, %7 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %8 row_newbcast:5 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]));
   return acc + odd;
 }
@@ -270,7 +272,7 @@ __device__ __forceinline__ float row_fma_seed(const float (&w)[12], float s, flo
       "v_fmac_f32_dpp %1, %2, %12 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %0, %2, %13 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %14 row_newbcast:11 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]));
   return acc + odd;
 }
@@ -291,7 +293,7 @@ __device__ __forceinline__ float row_fma_seed(const float (&w)[13], float s, flo
       "v_fmac_f32_dpp %0, %2, %13 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %14 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %0, %2, %15 row_newbcast:12 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]));
   return acc + odd;
 }
@@ -303,7 +305,7 @@ __device__ __forceinline__ double row_fma_seed(const double (&w)[4], double s, d
       "v_fmac_f64_dpp %1, %2, %4 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %5 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %6 row_newbcast:3 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]));
   return acc + odd;
 }
@@ -317,7 +319,7 @@ __device__ __forceinline__ double row_fma_seed(const double (&w)[6], double s, d
       "v_fmac_f64_dpp %1, %2, %6 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %7 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %8 row_newbcast:5 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]));
   return acc + odd;
 }
@@ -337,7 +339,7 @@ __device__ __forceinline__ double row_fma_seed(const double (&w)[12], double s, 
       "v_fmac_f64_dpp %1, %2, %12 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %13 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %14 row_newbcast:11 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]));
   return acc + odd;
 }
@@ -358,7 +360,7 @@ __device__ __forceinline__ double row_fma_seed(const double (&w)[13], double s, 
       "v_fmac_f64_dpp %0, %2, %13 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %14 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %15 row_newbcast:12 row_mask:0xf bank_mask:0xf"
-      : "+v"(acc), "+v"(odd)
+      : "+&v"(acc), "+&v"(odd)
       : "v"(s), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]));
   return acc + odd;
 }
@@ -379,7 +381,7 @@ __device__ __forceinline__ void row_fma_2(const float (&w0)[4], float s0, float&
       "v_fmac_f32_dpp %0, %2, %7 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %3, %11 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s0), "v"(s1), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]));
 }
 
@@ -399,7 +401,7 @@ __device__ __forceinline__ void row_fma_3(const float (&w0)[4], float s0, float&
       "v_fmac_f32_dpp %1, %4, %13 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %2, %5, %17 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1), "+v"(a2)
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2)
       : "v"(s0), "v"(s1), "v"(s2), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w2[0]), "v"(w2[1]), "v"(w2[2]), "v"(w2[3]));
 }
 
@@ -419,7 +421,7 @@ __device__ __forceinline__ void row_fma_2(const float (&w0)[6], float s0, float&
       "v_fmac_f32_dpp %0, %2, %9 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %3, %15 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s0), "v"(s1), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]));
 }
 
@@ -445,7 +447,7 @@ __device__ __forceinline__ void row_fma_3(const float (&w0)[6], float s0, float&
       "v_fmac_f32_dpp %1, %4, %17 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %2, %5, %23 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1), "+v"(a2)
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2)
       : "v"(s0), "v"(s1), "v"(s2), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w2[0]), "v"(w2[1]), "v"(w2[2]), "v"(w2[3]), "v"(w2[4]), "v"(w2[5]));
 }
 
@@ -477,7 +479,7 @@ __device__ __forceinline__ void row_fma_2(const float (&w0)[12], float s0, float
       "v_fmac_f32_dpp %0, %2, %15 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %3, %27 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s0), "v"(s1), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w0[6]), "v"(w0[7]), "v"(w0[8]), "v"(w0[9]), "v"(w0[10]), "v"(w0[11]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w1[6]), "v"(w1[7]), "v"(w1[8]), "v"(w1[9]), "v"(w1[10]), "v"(w1[11]));
 }
 
@@ -521,7 +523,7 @@ __device__ __forceinline__ void row_fma_3(const float (&w0)[12], float s0, float
       "v_fmac_f32_dpp %1, %4, %29 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %2, %5, %41 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1), "+v"(a2)
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2)
       : "v"(s0), "v"(s1), "v"(s2), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w0[6]), "v"(w0[7]), "v"(w0[8]), "v"(w0[9]), "v"(w0[10]), "v"(w0[11]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w1[6]), "v"(w1[7]), "v"(w1[8]), "v"(w1[9]), "v"(w1[10]), "v"(w1[11]), "v"(w2[0]), "v"(w2[1]), "v"(w2[2]), "v"(w2[3]), "v"(w2[4]), "v"(w2[5]), "v"(w2[6]), "v"(w2[7]), "v"(w2[8]), "v"(w2[9]), "v"(w2[10]), "v"(w2[11]));
 }
 
@@ -555,7 +557,7 @@ __device__ __forceinline__ void row_fma_2(const float (&w0)[13], float s0, float
       "v_fmac_f32_dpp %0, %2, %16 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %3, %29 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s0), "v"(s1), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w0[6]), "v"(w0[7]), "v"(w0[8]), "v"(w0[9]), "v"(w0[10]), "v"(w0[11]), "v"(w0[12]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w1[6]), "v"(w1[7]), "v"(w1[8]), "v"(w1[9]), "v"(w1[10]), "v"(w1[11]), "v"(w1[12]));
 }
 
@@ -602,7 +604,7 @@ __device__ __forceinline__ void row_fma_3(const float (&w0)[13], float s0, float
       "v_fmac_f32_dpp %1, %4, %31 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %2, %5, %44 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1), "+v"(a2)
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2)
       : "v"(s0), "v"(s1), "v"(s2), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w0[6]), "v"(w0[7]), "v"(w0[8]), "v"(w0[9]), "v"(w0[10]), "v"(w0[11]), "v"(w0[12]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w1[6]), "v"(w1[7]), "v"(w1[8]), "v"(w1[9]), "v"(w1[10]), "v"(w1[11]), "v"(w1[12]), "v"(w2[0]), "v"(w2[1]), "v"(w2[2]), "v"(w2[3]), "v"(w2[4]), "v"(w2[5]), "v"(w2[6]), "v"(w2[7]), "v"(w2[8]), "v"(w2[9]), "v"(w2[10]), "v"(w2[11]), "v"(w2[12]));
 }
 
@@ -616,7 +618,7 @@ __device__ __forceinline__ void row_fma_x2(float s, const float (&w0)[2], float&
       "v_fmac_f32_dpp %0, %2, %4 row_newbcast:%c8 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %6 row_newbcast:%c8 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s), "v"(w0[0]), "v"(w0[1]), "v"(w1[0]), "v"(w1[1]), "n"(O + 0), "n"(O + 1));
 }
 
@@ -632,7 +634,7 @@ __device__ __forceinline__ void row_fma_x2(float s, const float (&w0)[3], float&
       "v_fmac_f32_dpp %0, %2, %5 row_newbcast:%c11 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %8 row_newbcast:%c11 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "n"(O + 0), "n"(O + 1), "n"(O + 2));
 }
 
@@ -650,7 +652,7 @@ __device__ __forceinline__ void row_fma_x2(float s, const float (&w0)[4], float&
       "v_fmac_f32_dpp %0, %2, %6 row_newbcast:%c14 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f32_dpp %1, %2, %10 row_newbcast:%c14 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3));
 }
 
@@ -666,7 +668,7 @@ __device__ __forceinline__ void row_fma_2(const double (&w0)[4], double s0, doub
       "v_fmac_f64_dpp %0, %2, %7 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %3, %11 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s0), "v"(s1), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]));
 }
 
@@ -686,7 +688,7 @@ __device__ __forceinline__ void row_fma_3(const double (&w0)[4], double s0, doub
       "v_fmac_f64_dpp %1, %4, %13 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %2, %5, %17 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1), "+v"(a2)
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2)
       : "v"(s0), "v"(s1), "v"(s2), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w2[0]), "v"(w2[1]), "v"(w2[2]), "v"(w2[3]));
 }
 
@@ -706,7 +708,7 @@ __device__ __forceinline__ void row_fma_2(const double (&w0)[6], double s0, doub
       "v_fmac_f64_dpp %0, %2, %9 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %3, %15 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s0), "v"(s1), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]));
 }
 
@@ -732,7 +734,7 @@ __device__ __forceinline__ void row_fma_3(const double (&w0)[6], double s0, doub
       "v_fmac_f64_dpp %1, %4, %17 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %2, %5, %23 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1), "+v"(a2)
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2)
       : "v"(s0), "v"(s1), "v"(s2), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w2[0]), "v"(w2[1]), "v"(w2[2]), "v"(w2[3]), "v"(w2[4]), "v"(w2[5]));
 }
 
@@ -764,7 +766,7 @@ __device__ __forceinline__ void row_fma_2(const double (&w0)[12], double s0, dou
       "v_fmac_f64_dpp %0, %2, %15 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %3, %27 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s0), "v"(s1), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w0[6]), "v"(w0[7]), "v"(w0[8]), "v"(w0[9]), "v"(w0[10]), "v"(w0[11]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w1[6]), "v"(w1[7]), "v"(w1[8]), "v"(w1[9]), "v"(w1[10]), "v"(w1[11]));
 }
 
@@ -808,7 +810,7 @@ __device__ __forceinline__ void row_fma_3(const double (&w0)[12], double s0, dou
       "v_fmac_f64_dpp %1, %4, %29 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %2, %5, %41 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1), "+v"(a2)
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2)
       : "v"(s0), "v"(s1), "v"(s2), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w0[6]), "v"(w0[7]), "v"(w0[8]), "v"(w0[9]), "v"(w0[10]), "v"(w0[11]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w1[6]), "v"(w1[7]), "v"(w1[8]), "v"(w1[9]), "v"(w1[10]), "v"(w1[11]), "v"(w2[0]), "v"(w2[1]), "v"(w2[2]), "v"(w2[3]), "v"(w2[4]), "v"(w2[5]), "v"(w2[6]), "v"(w2[7]), "v"(w2[8]), "v"(w2[9]), "v"(w2[10]), "v"(w2[11]));
 }
 
@@ -842,7 +844,7 @@ __device__ __forceinline__ void row_fma_2(const double (&w0)[13], double s0, dou
       "v_fmac_f64_dpp %0, %2, %16 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %3, %29 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s0), "v"(s1), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w0[6]), "v"(w0[7]), "v"(w0[8]), "v"(w0[9]), "v"(w0[10]), "v"(w0[11]), "v"(w0[12]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w1[6]), "v"(w1[7]), "v"(w1[8]), "v"(w1[9]), "v"(w1[10]), "v"(w1[11]), "v"(w1[12]));
 }
 
@@ -889,7 +891,7 @@ __device__ __forceinline__ void row_fma_3(const double (&w0)[13], double s0, dou
       "v_fmac_f64_dpp %1, %4, %31 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %2, %5, %44 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1), "+v"(a2)
+      : "+&v"(a0), "+&v"(a1), "+&v"(a2)
       : "v"(s0), "v"(s1), "v"(s2), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w0[4]), "v"(w0[5]), "v"(w0[6]), "v"(w0[7]), "v"(w0[8]), "v"(w0[9]), "v"(w0[10]), "v"(w0[11]), "v"(w0[12]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "v"(w1[4]), "v"(w1[5]), "v"(w1[6]), "v"(w1[7]), "v"(w1[8]), "v"(w1[9]), "v"(w1[10]), "v"(w1[11]), "v"(w1[12]), "v"(w2[0]), "v"(w2[1]), "v"(w2[2]), "v"(w2[3]), "v"(w2[4]), "v"(w2[5]), "v"(w2[6]), "v"(w2[7]), "v"(w2[8]), "v"(w2[9]), "v"(w2[10]), "v"(w2[11]), "v"(w2[12]));
 }
 
@@ -903,7 +905,7 @@ __device__ __forceinline__ void row_fma_x2(double s, const double (&w0)[2], doub
       "v_fmac_f64_dpp %0, %2, %4 row_newbcast:%c8 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %6 row_newbcast:%c8 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s), "v"(w0[0]), "v"(w0[1]), "v"(w1[0]), "v"(w1[1]), "n"(O + 0), "n"(O + 1));
 }
 
@@ -919,7 +921,7 @@ __device__ __forceinline__ void row_fma_x2(double s, const double (&w0)[3], doub
       "v_fmac_f64_dpp %0, %2, %5 row_newbcast:%c11 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %8 row_newbcast:%c11 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "n"(O + 0), "n"(O + 1), "n"(O + 2));
 }
 
@@ -937,7 +939,7 @@ __device__ __forceinline__ void row_fma_x2(double s, const double (&w0)[4], doub
       "v_fmac_f64_dpp %0, %2, %6 row_newbcast:%c14 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %10 row_newbcast:%c14 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(s), "v"(w0[0]), "v"(w0[1]), "v"(w0[2]), "v"(w0[3]), "v"(w1[0]), "v"(w1[1]), "v"(w1[2]), "v"(w1[3]), "n"(O + 0), "n"(O + 1), "n"(O + 2), "n"(O + 3));
 }
 
@@ -951,7 +953,7 @@ __device__ __forceinline__ void row_axpy(double (&c)[4], double src, double s) {
       "v_fmac_f64_dpp %2, %4, %5 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %3, %4, %5 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3])
+      : "+&v"(c[0]), "+&v"(c[1]), "+&v"(c[2]), "+&v"(c[3])
       : "v"(src), "v"(s));
 }
 
@@ -965,7 +967,7 @@ __device__ __forceinline__ void row_axpy(double (&c)[6], double src, double s) {
       "v_fmac_f64_dpp %4, %6, %7 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %5, %6, %7 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5])
+      : "+&v"(c[0]), "+&v"(c[1]), "+&v"(c[2]), "+&v"(c[3]), "+&v"(c[4]), "+&v"(c[5])
       : "v"(src), "v"(s));
 }
 
@@ -985,7 +987,7 @@ __device__ __forceinline__ void row_axpy(double (&c)[12], double src, double s) 
       "v_fmac_f64_dpp %10, %12, %13 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %11, %12, %13 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5]), "+v"(c[6]), "+v"(c[7]), "+v"(c[8]), "+v"(c[9]), "+v"(c[10]), "+v"(c[11])
+      : "+&v"(c[0]), "+&v"(c[1]), "+&v"(c[2]), "+&v"(c[3]), "+&v"(c[4]), "+&v"(c[5]), "+&v"(c[6]), "+&v"(c[7]), "+&v"(c[8]), "+&v"(c[9]), "+&v"(c[10]), "+&v"(c[11])
       : "v"(src), "v"(s));
 }
 
@@ -1006,7 +1008,7 @@ __device__ __forceinline__ void row_axpy(double (&c)[13], double src, double s) 
       "v_fmac_f64_dpp %11, %13, %14 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %12, %13, %14 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5]), "+v"(c[6]), "+v"(c[7]), "+v"(c[8]), "+v"(c[9]), "+v"(c[10]), "+v"(c[11]), "+v"(c[12])
+      : "+&v"(c[0]), "+&v"(c[1]), "+&v"(c[2]), "+&v"(c[3]), "+&v"(c[4]), "+&v"(c[5]), "+&v"(c[6]), "+&v"(c[7]), "+&v"(c[8]), "+&v"(c[9]), "+&v"(c[10]), "+&v"(c[11]), "+&v"(c[12])
       : "v"(src), "v"(s));
 }
 
@@ -1022,7 +1024,7 @@ __device__ __forceinline__ void row_sweep(double (&a)[4], double g) {
       "v_fmac_f64_dpp %2, %2, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %3, %3, %4 row_newbcast:%c5 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3])
+      : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3])
       : "v"(g), "n"(KP));
 }
 
@@ -1037,7 +1039,7 @@ __device__ __forceinline__ void row_sweep(double (&a)[6], double g) {
       "v_fmac_f64_dpp %4, %4, %6 row_newbcast:%c7 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %5, %5, %6 row_newbcast:%c7 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5])
+      : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5])
       : "v"(g), "n"(KP));
 }
 
@@ -1058,7 +1060,7 @@ __device__ __forceinline__ void row_sweep(double (&a)[12], double g) {
       "v_fmac_f64_dpp %10, %10, %12 row_newbcast:%c13 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %11, %11, %12 row_newbcast:%c13 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11])
+      : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7]), "+&v"(a[8]), "+&v"(a[9]), "+&v"(a[10]), "+&v"(a[11])
       : "v"(g), "n"(KP));
 }
 
@@ -1080,7 +1082,7 @@ __device__ __forceinline__ void row_sweep(double (&a)[13], double g) {
       "v_fmac_f64_dpp %11, %11, %13 row_newbcast:%c14 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %12, %12, %13 row_newbcast:%c14 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]), "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), "+v"(a[12])
+      : "+&v"(a[0]), "+&v"(a[1]), "+&v"(a[2]), "+&v"(a[3]), "+&v"(a[4]), "+&v"(a[5]), "+&v"(a[6]), "+&v"(a[7]), "+&v"(a[8]), "+&v"(a[9]), "+&v"(a[10]), "+&v"(a[11]), "+&v"(a[12])
       : "v"(g), "n"(KP));
 }
 

@@ -145,7 +145,7 @@ __device__ __forceinline__ double dot_pair(const double (&w)[6], const RowPair<d
       "v_fmac_f64_dpp %0, %2, %8 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %9 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(v.x), "v"(v.y), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]));
   return a0 + a1;
 }
@@ -164,7 +164,7 @@ __device__ __forceinline__ double dot_pair(const double (&w)[9], const RowPair<d
       "v_fmac_f64_dpp %1, %2, %11 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %2, %12 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(v.x), "v"(v.y), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]));
   return a0 + a1;
 }
@@ -190,7 +190,7 @@ __device__ __forceinline__ double dot_pair(const double (&w)[16], const RowPair<
       "v_fmac_f64_dpp %0, %2, %18 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %2, %19 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(v.x), "v"(v.y), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]), "v"(w[13]), "v"(w[14]), "v"(w[15]));
   return a0 + a1;
 }
@@ -217,7 +217,7 @@ __device__ __forceinline__ double dot_pair(const double (&w)[17], const RowPair<
       "v_fmac_f64_dpp %1, %2, %19 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %3, %20 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(v.x), "v"(v.y), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]), "v"(w[13]), "v"(w[14]), "v"(w[15]), "v"(w[16]));
   return a0 + a1;
 }
@@ -303,7 +303,7 @@ __device__ __forceinline__ double dot_pair(const double (&w)[32], const RowPair<
       "v_fmac_f64_dpp %0, %3, %34 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %1, %3, %35 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
       "s_nop 1"
-      : "+v"(a0), "+v"(a1)
+      : "+&v"(a0), "+&v"(a1)
       : "v"(v.x), "v"(v.y), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]), "v"(w[13]), "v"(w[14]), "v"(w[15]), "v"(w[16]), "v"(w[17]), "v"(w[18]), "v"(w[19]), "v"(w[20]), "v"(w[21]), "v"(w[22]), "v"(w[23]), "v"(w[24]), "v"(w[25]), "v"(w[26]), "v"(w[27]), "v"(w[28]), "v"(w[29]), "v"(w[30]), "v"(w[31]));
   return a0 + a1;
 }
