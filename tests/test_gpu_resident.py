@@ -182,3 +182,32 @@ def test_resident_factor_one_and_two_wavefronts(shape):
     torch.cuda.synchronize()
     for k in FIELDS:
         assert torch.equal(getattr(outs[0], k)[:7], getattr(outs[1], k)), k
+
+
+@pytest.mark.parametrize("horizon", [50, 20])
+def test_resident_is_as_near_to_64_bits_as_the_streaming_kernel(horizon):
+    """fp32, 100 iterations: per output, the distance from the fp64 solve of the same
+    data is no larger than the streaming kernel's, whose sums have as many roundings at
+    the size of the duals (1.15: two draws of such errors over 64 problems)."""
+    from turbompc_amd.problems import configs
+
+    prob = configs.config2(B=64, seed=2)
+    qp = prob.build_qp(*prob.initial_guess()).to("cpu", torch.float32).to("cpu", torch.float64)
+    cut = lambda t, k: t[:, :horizon + k].contiguous()  # noqa: E731
+    qp = dataclasses.replace(
+        qp, cost=dataclasses.replace(qp.cost, D=cut(qp.cost.D, 1), E=cut(qp.cost.E, 0), q=cut(qp.cost.q, 1)),
+        eq=dataclasses.replace(qp.eq, A_minus=cut(qp.eq.A_minus, 0), A_plus=cut(qp.eq.A_plus, 0), c=cut(qp.eq.c, 0)),
+        ineq=dataclasses.replace(qp.ineq, **{k: cut(getattr(qp.ineq, k), 1) for k in ("G", "l", "u")}))
+    cfg = _cfg(max_iter=100, check_every=101, alpha=1.0)
+    run = lambda dtype, **kw: _solver(qp, cfg, std_dynamics=True, diag_cost=True, **kw).solve(  # noqa: E731
+        qp.to(DEV, dtype), _state_to_dev(zero_state(qp, 0.1), dtype))[2]
+    exact, chip, stream = run(torch.float64), run(torch.float32), run(torch.float32, kernel_flags=_lib.flag_stream_p(1))
+    torch.cuda.synchronize()
+    nx = 12
+    parts = {"states": lambda s: s.x_blocks[..., :nx], "controls": lambda s: s.x_blocks[..., nx:], "z_g": lambda s: s.z_g,
+             "y_g": lambda s: s.y_g, "y_f_0": lambda s: s.y_f_0, "y_f_dyn": lambda s: s.y_f_dyn}
+    for name, f in parts.items():
+        e, err = f(exact), lambda s: float((f(s).double() - e).norm() / e.norm())  # noqa: E731,B023
+        a, b = err(chip), err(stream)
+        print(f"  T = {horizon + 1}, {name}: on-chip {a:.2e}, streaming {b:.2e}", flush=True)
+        assert a < 1.15 * b, name
