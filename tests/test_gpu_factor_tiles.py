@@ -63,3 +63,33 @@ def test_adjoint_sweeps_of_34_rows(dims):
     for flags in (0, _lib.FLAG_GENERIC_KERNEL):
         dz, mult = solve_backward_kkt_hip(qd, refine_steps=4, kernel_flags=flags)
         assert rel_err(dz, dz_ref) < 1e-9 and rel_err(mult, mult_ref) < 1e-9
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("n", [1, 6, 9, 16, 17, 34])
+def test_blktri_infinite_pivot_pins_its_variable(n, dtype):
+    """An infinite diagonal entry: its variable is zero, the others solve the system
+    without its row and column."""
+    B, T = 3, 5
+    S, rhs = _system(B, T, n, seed=200 + n)
+    pins = [(1, n - 1), (3, n // 2)]
+    for t, i in pins:
+        S[:, t, i, n + i] = np.inf
+    x = hip_blktri_solve(torch.tensor(S, dtype=dtype, device=DEV), torch.tensor(rhs, dtype=dtype, device=DEV))
+    keep = np.setdiff1d(np.arange(T * n), [t * n + i for t, i in pins])
+    want = np.zeros((B, T * n))
+    for b in range(B):
+        want[b, keep] = np.linalg.solve(blocks_to_dense(S[b])[np.ix_(keep, keep)], rhs[b].reshape(-1)[keep])
+    assert rel_err(x, want.reshape(B, T, n)) < TOL[dtype]
+    for t, i in pins:
+        assert bool((x[:, t, i] == 0).all())
+
+
+@pytest.mark.parametrize("n", [6, 16, 34])
+def test_blktri_scaled_by_powers_of_two(n):
+    """S and the right-hand side scaled towards the ends of the range: the same x."""
+    S, rhs = _system(2, 5, n, seed=300 + n)
+    x = hip_blktri_solve(torch.tensor(S, device=DEV), torch.tensor(rhs, device=DEV))
+    for e in (-1010, -700, 700, 1010):
+        y = hip_blktri_solve(torch.tensor(np.ldexp(S, e), device=DEV), torch.tensor(np.ldexp(rhs, e), device=DEV))
+        assert rel_err(y, x) < 1e-12, e
