@@ -550,7 +550,7 @@ __global__ __launch_bounds__(TPB, WPE) void admm_resident_kernel(ResArgs<R> a) {
         ld_row(c[(k + CB - 1) % CB], q + (k + CB - 1) * CW);
         q[k * CW + CX + lr] = r;
         // (gx and h first: each alone is as large as the duals, and would be rounded so with
-        // every term: fp32, T = 51, NX = 12 states 1.29e-6 off 64 bits, 6.5e-7 like this)
+        // every term: fp32, T = 51, NX = 12 states 1.29e-6 off 64 bits, 7.1e-7 like this)
         r = row_fma<0>(c[k].w, r, c[(k + 1) % CB].g + c[(k + 1) % CB].h);
       };
       int p = mid;
