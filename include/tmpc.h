@@ -108,8 +108,8 @@ typedef struct tmpc_state {
  * dynamics: D, E, q, G, l, u, A0, c0 and the slack weight are unchanged).  Only
  * the A_minus and c records are rewritten.  Vouched for by the caller; the
  * other paths ignore it: the on-chip path keeps no records and reads the whole
- * QP, and a streaming call of dims that the on-chip path takes under other
- * flags packs its records anew. */
+ * QP, and a streaming call after an on-chip call on the workspace packs its
+ * records anew. */
 #define TMPC_FLAG_WARM_RECORDS 8u
 /* With TMPC_FLAG_WARM_RECORDS: the QP also differs from the previous call's in
  * G, l and u (inequality rows relinearized at the new iterate, as the obstacle

@@ -162,6 +162,35 @@ def test_resident_leaves_no_warm_records():
             assert torch.equal(getattr(out, k), getattr(want, k)), (warm, k)
 
 
+@pytest.mark.parametrize("form", ["problems per wavefront", "lane groups", "invariant A"])
+@pytest.mark.parametrize("after", ["streaming", "on-chip", "generic"])
+def test_streaming_forms_keep_their_warm_records(form, after):
+    """Flags that keep a shape of the on-chip path on the streaming kernel: a warm call
+    keeps the records of a streaming call before it (a q that changed against the
+    caller's promise is not read) and packs them anew after a call of another path."""
+    from turbompc_amd.solvers.admm.admm_hip_backend import direct_workspace
+
+    qp = random_qp(6, 9, 17, 13, 4, seed=97, std=True, diag=True)
+    G = qp.ineq.G[:1, :1].expand_as(qp.ineq.G).contiguous()
+    qp = dataclasses.replace(qp, ineq=dataclasses.replace(qp.ineq, G=G))
+    kw = {"problems per wavefront": dict(kernel_flags=_lib.flag_stream_p(1)),
+          "lane groups": dict(kernel_flags=_lib.FLAG_FACTOR_GROUPS), "invariant A": dict(invariant_a=True)}[form]
+    solver = lambda **k: _solver(qp, _cfg(max_iter=8), std_dynamics=True, diag_cost=True, const_g=True, **k)  # noqa: E731
+    stream = solver(**kw)
+    first = {"streaming": stream, "on-chip": solver(), "generic": solver(kernel_flags=_lib.FLAG_GENERIC_KERNEL)}[after]
+    st0 = _state_to_dev(zero_state(qp, 0.1), torch.float64)
+    qpd = qp.to(DEV, torch.float64)
+    other = dataclasses.replace(qpd, cost=dataclasses.replace(qpd.cost, q=qpd.cost.q + 1.0))
+    active = torch.ones(6, dtype=torch.bool, device=DEV)
+    ws = direct_workspace(qpd)
+    (_, _), _, mid = first.solve(qpd, st0, workspace=ws)
+    (_, _), _, got, _, _ = stream.sqp_step(other, mid, active, None, workspace=ws, warm_records=True)
+    (_, _), _, want, _, _ = stream.sqp_step(qpd if after == "streaming" else other, mid, active, None)
+    torch.cuda.synchronize()
+    for k in FIELDS:
+        assert torch.equal(getattr(got, k), getattr(want, k)), k
+
+
 @pytest.mark.parametrize("shape", [(5, 17, 13, 4), (6, 9, 6, 11), (4, 16, 12, 9)])
 def test_resident_factor_one_and_two_wavefronts(shape):
     """The factorization with a wavefront of its own for the preparation (up to 1024

@@ -304,13 +304,16 @@ __device__ __forceinline__ int kth_set_bit(uint32_t x, int k) {
 // 1 + sigma and the iteration keeps them at zero without touching any other
 // value.  With A0p, the wavefront of (b, 0) also writes the problem's A0 with
 // rows of n entries.
+// With held, nothing is packed where the workspace says that it holds the records.
 constexpr int kPackWaves = 4;
 
 template <typename R>
 __global__ __launch_bounds__(kWave * kPackWaves) void stage_pack_kernel(Dims d, QPDev<R> qp, StateDev<R> st,
                                                                         R* __restrict__ am, R* __restrict__ rv,
                                                                         R* __restrict__ dm, int diag,
-                                                                        R* __restrict__ A0p) {
+                                                                        R* __restrict__ A0p,
+                                                                        const uint32_t* __restrict__ held) {
+  if (held != nullptr && held[kRecordsWord] == kRecordsHeld) return;
   const int b = blockIdx.x * kPackWaves + (int)(threadIdx.x / kWave), t = blockIdx.y;
   const int tid = (int)(threadIdx.x % kWave);
   const int B = d.B, T = d.T, N = d.N, n = d.n, nx = d.nx, m = d.m, nq = d.nq;
@@ -462,11 +465,13 @@ __global__ __launch_bounds__(256) void stage_repack_dynamics_kernel(Dims d, cons
 // y_f0 and rho, which the iteration kernel writes directly.  A problem's flag
 // is set by atomicOr from each block that meets one of its non-finite values
 // (the result does not depend on their order).
+// The call's last kernel also notes in the workspace that it holds the records.
 constexpr int kUnpackProblems = 32;
 
 template <typename R>
 __global__ __launch_bounds__(256) void stage_unpack_kernel(Dims d, const R* __restrict__ rv, StateDev<R> st,
-                                                           uint32_t* __restrict__ iters) {
+                                                           uint32_t* __restrict__ iters, uint32_t* __restrict__ held) {
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) held[kRecordsWord] = kRecordsHeld;
   __shared__ uint32_t bad[kUnpackProblems];
   const int t = blockIdx.y, b0 = blockIdx.x * kUnpackProblems;
   const int B = d.B, T = d.T, N = d.N, n = d.nq, nx = d.nx, m = d.m;  // n: the state's row length

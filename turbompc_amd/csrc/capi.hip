@@ -573,7 +573,8 @@ StreamArgs<R> stream_args(const AdmmArgs<R>& a, const DirectWs<R>& w, const Dims
 }
 
 // The on-chip path's part of the workspace (resident_api.hpp), in place of the
-// stage records: the factor, then the control words and residuals.
+// stage records: the control words (the first problem's fourth: kRecordsWord), the
+// factor, the residuals.
 template <typename R>
 struct ResidentWs {
   R *V, *L, *res;
@@ -590,9 +591,9 @@ template <typename R>
 ResidentWs<R> carve_resident(void* ws, const Dims& d, int cls) {
   Carver c{static_cast<char*>(ws)};
   ResidentWs<R> w;
+  w.ctl = c.take<int32_t>((size_t)d.B * 4);
   w.V = reinterpret_cast<R*>(c.take<char>(resident_v_bytes(d, sizeof(R), cls)));
   w.L = reinterpret_cast<R*>(c.take<char>(resident_l_bytes(d, sizeof(R), cls)));
-  w.ctl = c.take<int32_t>((size_t)d.B * 4);
   w.res = c.take<R>((size_t)d.B * 8);
   return w;
 }
@@ -768,10 +769,12 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
   const ResPlan rp = other_form ? ResPlan{} : res_plan(const_g);
   const bool resident = rp.cls >= 0;
   const bool stream = !resident && streamable && (cfg->flags & TMPC_FLAG_GENERIC_KERNEL) == 0;
-  // Warm stage records: the previous call on the workspace left them, unless these
-  // dims run on-chip under other flags (the plan with one G takes the least LDS):
-  // that path keeps no records, so they are packed anew.
-  const bool warm = (cfg->flags & TMPC_FLAG_WARM_RECORDS) != 0 && res_plan(true).cls < 0;
+  // Warm stage records: the previous call on the workspace left them, unless it ran
+  // on-chip (which these dims can under other flags; the plan with one G takes the
+  // least LDS).  That path keeps none, so the pack kernel then looks (held).
+  const bool warm = (cfg->flags & TMPC_FLAG_WARM_RECORDS) != 0;
+  const bool maybe_cold = warm && stream && res_plan(true).cls >= 0;
+  uint32_t* held = static_cast<uint32_t*>(ws);
   // the AINV form: asked for, with the resident G rows, at most two problems
   // per wavefront, and the whole workspace
   const bool ainv = stream && const_g && (cfg->flags & TMPC_FLAG_INVARIANT_A) != 0 && ainv_shape_ok(dr, sizeof(R)) && sp <= 2 &&
@@ -839,6 +842,13 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
     if (st) return st;
     a.act = sq->active_out;
   }
+  if (stream && (!warm || maybe_cold)) {
+    hipLaunchKernelGGL((stage_pack_kernel<R>), dim3((unsigned)((d.B + kPackWaves - 1) / kPackWaves), (unsigned)d.T),
+                       dim3(kWave * kPackWaves), 0, s, dr, a.qp, a.st, w.am, w.rv, w.dm, diag ? 1 : 0,
+                       pad ? w.a0p : (R*)nullptr, warm ? held : nullptr);
+    st = launch_status();
+    if (st) return st;
+  }
   if (stream && warm) {
     const unsigned gx = (unsigned)((d.B + kRepackProblems - 1) / kRepackProblems);
     // the A_minus and c rows are rewritten unless they did not change or the
@@ -852,12 +862,6 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
     else if (dyn_rows)
       hipLaunchKernelGGL((stage_repack_dynamics_kernel<R, false>), dim3(gx, (unsigned)d.N), dim3(256), 0, s, dr,
                          a.qp.Am, a.qp.c, a.qp.G, a.qp.l, a.qp.u, w.am, w.rv, diag ? 1 : 0, 1);
-    st = launch_status();
-    if (st) return st;
-  } else if (stream) {
-    hipLaunchKernelGGL((stage_pack_kernel<R>), dim3((unsigned)((d.B + kPackWaves - 1) / kPackWaves), (unsigned)d.T),
-                       dim3(kWave * kPackWaves), 0, s, dr, a.qp, a.st, w.am, w.rv, w.dm, diag ? 1 : 0,
-                       pad ? w.a0p : (R*)nullptr);
     st = launch_status();
     if (st) return st;
   }
@@ -930,7 +934,7 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
   if (stream) {  // the unpack also sets the non-finite flags
     hipLaunchKernelGGL((stage_unpack_kernel<R>),
                        dim3((unsigned)((d.B + kUnpackProblems - 1) / kUnpackProblems), (unsigned)d.T), dim3(256), 0,
-                       s, dr, (const R*)w.rv, a.st, iters);
+                       s, dr, (const R*)w.rv, a.st, iters, held);
     return launch_status();
   }
   return launch_nonfinite_flags<R>(s, d, a.st, iters);

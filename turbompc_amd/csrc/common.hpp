@@ -44,6 +44,14 @@ __host__ __device__ __forceinline__ constexpr int packed_size(int n) { return (n
 // consecutive problems load as one run of 128-bit accesses.
 __host__ __device__ __forceinline__ constexpr int th_pitch(int n) { return (packed_size(n) + 3) & ~3; }
 
+// What a workspace of the direct solve holds between calls: word kRecordsWord is
+// kRecordsHeld after a streaming call (whose stage records a warm call keeps) and
+// something else after any other.  The streaming and generic paths have the factor
+// there, which no later call reads (a NaN of this payload is no value of theirs), the
+// on-chip path a control word of its own that it clears.
+constexpr int kRecordsWord = 3;
+constexpr uint32_t kRecordsHeld = 0xfff9c0deu;
+
 // `it % k == 0` with XLA's integer remainder convention (x % 0 == x), which is
 // what the reference's jnp expressions evaluate to when k == 0.
 __device__ __forceinline__ bool mod_zero(int it, int k) {

@@ -221,6 +221,7 @@ __global__ __launch_bounds__(TPB, WPE) void admm_resident_kernel(ResArgs<R> a) {
     if (wrote && r0l) a.y_f0[(size_t)b * n0 + zr] = y0;
     const bool any = __syncthreads_or(bad ? 1 : 0) != 0;
     if (tid == 0) {
+      if (b == 0) a.ctl[kRecordsWord] = 0;
       a.ctl[b * 4 + 0] = it;
       a.ctl[b * 4 + 1] = done ? 1 : 0;
       const bool turned = rho != rho_in;
