@@ -23,12 +23,24 @@ def _cfg(**kw):
     return oracle.OracleCfg(**base)
 
 
+def _first(qp, k):
+    """The batch's first k problems."""
+    cut = lambda p: dataclasses.replace(p, **{  # noqa: E731
+        f.name: getattr(p, f.name)[:k] for f in dataclasses.fields(p)
+        if torch.is_tensor(getattr(p, f.name)) and getattr(p, f.name).ndim > 0})
+    return dataclasses.replace(qp, **{f.name: cut(getattr(qp, f.name)) for f in dataclasses.fields(qp)
+                                      if dataclasses.is_dataclass(getattr(qp, f.name))})
+
+
 # (B, T, n, nx, m): n0 = nx; exact and padded classes, odd and even horizons
 SHAPES = [(3, 2, 6, 4, 2), (5, 3, 6, 4, 4), (4, 64, 6, 4, 2), (3, 17, 4, 3, 1), (2, 21, 2, 1, 0),
           (3, 2, 9, 6, 3), (4, 33, 9, 6, 4), (2, 101, 9, 6, 3), (3, 13, 8, 5, 2),
           (3, 13, 9, 6, 11), (2, 61, 9, 6, 11), (3, 8, 8, 6, 12), (3, 9, 9, 6, 5),
           (3, 9, 16, 12, 16), (2, 22, 16, 12, 16), (3, 11, 13, 10, 13), (2, 10, 14, 10, 0),
           (3, 2, 17, 13, 4), (2, 33, 17, 13, 4), (2, 34, 17, 13, 3), (3, 12, 15, 13, 2)]
+# horizons around the steps of the wavefront count, with more than hold the stages
+SHAPES += [(2, 12, 17, 13, 4), (2, 24, 17, 13, 4), (2, 31, 17, 13, 4), (2, 41, 6, 4, 2), (2, 33, 9, 6, 11),
+           (2, 57, 9, 6, 3), (2, 15, 16, 12, 16), (2, 29, 9, 6, 4)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
@@ -191,22 +203,18 @@ def test_streaming_forms_keep_their_warm_records(form, after):
         assert torch.equal(getattr(got, k), getattr(want, k)), k
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("shape", [(5, 17, 13, 4), (6, 9, 6, 11), (4, 16, 12, 9)])
-def test_resident_factor_one_and_two_wavefronts(shape):
+def test_resident_factor_one_and_two_wavefronts(shape, dtype):
     """The factorization with a wavefront of its own for the preparation (up to 1024
     problems) and without: the same bits."""
     T, n, nx, m = shape
     qp = random_qp(1026, T, n, nx, m, seed=96, std=True, diag=True)
-    part = type(qp)(**{f.name: getattr(qp, f.name) for f in dataclasses.fields(qp)})
-    part = dataclasses.replace(
-        part, **{f.name: dataclasses.replace(getattr(qp, f.name), **{
-            g.name: getattr(getattr(qp, f.name), g.name)[:7] for g in dataclasses.fields(getattr(qp, f.name))
-            if torch.is_tensor(getattr(getattr(qp, f.name), g.name)) and getattr(getattr(qp, f.name), g.name).ndim > 0})
-            for f in dataclasses.fields(qp) if dataclasses.is_dataclass(getattr(qp, f.name))})
+    part = _first(qp, 7)
     outs = []
     for q in (qp, part):
-        st = _state_to_dev(zero_state(q, 0.1), torch.float64)
-        (_, _), _, out = _solver(q, _cfg(), std_dynamics=True, diag_cost=True).solve(q.to(DEV, torch.float64), st)
+        st = _state_to_dev(zero_state(q, 0.1), dtype)
+        (_, _), _, out = _solver(q, _cfg(), std_dynamics=True, diag_cost=True).solve(q.to(DEV, dtype), st)
         outs.append(out)
     torch.cuda.synchronize()
     for k in FIELDS:
@@ -240,3 +248,32 @@ def test_resident_is_as_near_to_64_bits_as_the_streaming_kernel(horizon):
         a, b = err(chip), err(stream)
         print(f"  T = {horizon + 1}, {name}: on-chip {a:.2e}, streaming {b:.2e}", flush=True)
         assert a < 1.15 * b, name
+
+
+# (T, n, nx, m, const_g, slack) of the fp32 form with two workgroups per CU, which more than
+# 256 problems take: odd and even horizons, m below and at the class's, its largest horizons
+TWO_PER_CU = [(13, 9, 6, 11, False, False), (16, 9, 6, 12, False, True), (33, 9, 6, 11, False, True),
+              (64, 9, 6, 12, False, False), (12, 17, 13, 4, False, False), (25, 17, 13, 3, False, True),
+              (37, 17, 13, 4, False, False), (41, 17, 13, 4, True, False)]
+
+
+@pytest.mark.parametrize("case", TWO_PER_CU)
+def test_resident_two_workgroups_per_cu(case):
+    """fp32 against the oracle, and the first problems against a batch of their own, which
+    runs one workgroup per CU: the same bits."""
+    T, n, nx, m, const_g, slack = case
+    B = 259
+    qp = random_qp(B, T, n, nx, m, seed=98, std=True, diag=True)
+    if slack:
+        qp = soften(qp, 20.0, shrink=0.3)
+    if const_g:
+        G = qp.ineq.G[:1, :1].expand_as(qp.ineq.G).contiguous()
+        qp = dataclasses.replace(qp, ineq=dataclasses.replace(qp.ineq, G=G))
+    kw = dict(std_dynamics=True, diag_cost=True, const_g=const_g, use_slack=slack)
+    print(case, flush=True)
+    ref, it_ref, _, out, stats = _run_pair(qp, _cfg(), torch.float32, **kw)
+    np.testing.assert_array_equal(stats.num_iter.cpu().numpy(), it_ref)
+    _assert_state_close(out, ref, TOL[torch.float32])
+    _, _, _, few, _ = _run_pair(_first(qp, 7), _cfg(), torch.float32, **kw)
+    for k in FIELDS:
+        assert torch.equal(getattr(out, k)[:7], getattr(few, k)), k

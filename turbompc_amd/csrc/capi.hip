@@ -4,6 +4,7 @@
 #include "../../include/tmpc.h"
 
 #include <algorithm>
+#include <climits>
 #include <mutex>
 #include <vector>
 
@@ -753,27 +754,29 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
   if (stream_wide(dr) && (cfg->flags & TMPC_FLAG_STREAM_P(3)) == 0)
     sp = std::min(sp, kWave / stream_wide_rows(dr));  // the wide forms' groups are larger
   const bool streamable = std_dyn && stream_ok<R>(dr, sp, diag);
+  const std::vector<int> bounds = chunk_bounds(cfg->max_iter, cfg->check_every, cfg->adapt_rho_every);
   // The on-chip path: explicit-integrator structure, diagonal costs, a shape class
-  // whose blocks fit a workgroup, a factor that fits the records' room, and a batch
-  // for which it is the faster one (resident_pays).  A flag that asks for a form of
-  // the streaming or generic kernels keeps those.
-  auto res_plan = [&](bool cg) {
+  // whose blocks fit a workgroup, a factor that fits the records' room, and a batch and
+  // iterations for which it is the faster one (resident_pays).  A flag that asks for a
+  // form of the streaming or generic kernels keeps those.
+  auto res_plan = [&](bool cg, int iters, int chunks) {
     const ResPlan p = std_dyn && diag ? resident_plan(d, sizeof(R), cg) : ResPlan{};
     const bool runs = p.cls >= 0 && resident_ws_bytes<R>(d, p.cls) <= wsb &&
-                      (resident_pays(p.cls, d.B, sizeof(R)) || !streamable);
+                      (resident_pays(p, d, sizeof(R), iters, chunks) || !streamable);
     return runs ? p : ResPlan{};
   };
   constexpr uint32_t kOtherForm = TMPC_FLAG_GENERIC_KERNEL | TMPC_FLAG_FACTOR_GROUPS | TMPC_FLAG_STREAM_P(3);
   const bool other_form = (cfg->flags & kOtherForm) != 0 ||
                           (cfg->flags & (TMPC_FLAG_INVARIANT_A | TMPC_FLAG_ANY_FORM)) == TMPC_FLAG_INVARIANT_A;
-  const ResPlan rp = other_form ? ResPlan{} : res_plan(const_g);
+  const ResPlan rp = other_form ? ResPlan{} : res_plan(const_g, bounds.back(), (int)bounds.size() - 1);
   const bool resident = rp.cls >= 0;
   const bool stream = !resident && streamable && (cfg->flags & TMPC_FLAG_GENERIC_KERNEL) == 0;
   // Warm stage records: the previous call on the workspace left them, unless it ran
-  // on-chip (which these dims can under other flags; the plan with one G takes the
-  // least LDS).  That path keeps none, so the pack kernel then looks (held).
+  // on-chip (which these dims can under other flags or iteration counts; a plan with one
+  // G and many iterations is the likeliest).  That path keeps none, so the pack kernel
+  // then looks (held).
   const bool warm = (cfg->flags & TMPC_FLAG_WARM_RECORDS) != 0;
-  const bool maybe_cold = warm && stream && res_plan(true).cls >= 0;
+  const bool maybe_cold = warm && stream && res_plan(true, INT_MAX, 1).cls >= 0;
   uint32_t* held = static_cast<uint32_t*>(ws);
   // the AINV form: asked for, with the resident G rows, at most two problems
   // per wavefront, and the whole workspace
@@ -905,7 +908,6 @@ int admm_direct_impl(hipStream_t s, const tmpc_dims* dims, const tmpc_qp* qp,
     st = launch_ainv(s);
     if (st) return st;
   }
-  const std::vector<int> bounds = chunk_bounds(cfg->max_iter, cfg->check_every, cfg->adapt_rho_every);
   if (g_iter_events[0] && hipEventRecord(g_iter_events[0], s) != hipSuccess) return TMPC_ELAUNCH;
   for (size_t c = 0; c + 1 < bounds.size(); ++c) {
     if (c > 0) {

@@ -8,9 +8,9 @@
 namespace tmpc {
 
 // How a problem runs on the on-chip path: the shape class, wavefronts per
-// workgroup and LDS bytes; cls < 0: it does not.
+// workgroup, workgroups a CU holds and LDS bytes; cls < 0: it does not.
 struct ResPlan {
-  int cls = -1, nw = 0;
+  int cls = -1, nw = 0, per_cu = 0;
   bool dense = false;  // the form of which two workgroups share a CU
   size_t lds = 0;
 };
@@ -19,8 +19,9 @@ struct ResPlan {
 int resident_class(const Dims& d);
 // The plan for elements of elem bytes; const_g: one G for all stages and problems.
 ResPlan resident_plan(const Dims& d, size_t elem, bool const_g);
-// Whether the path beats the streaming kernel at B problems of the class.
-bool resident_pays(int cls, int B, size_t elem);
+// Whether the path beats the streaming kernel at d.B problems: iters iterations in
+// chunks chunks (a refactorization between them).
+bool resident_pays(const ResPlan& p, const Dims& d, size_t elem, int iters, int chunks);
 // Bytes of the factor arrays V and L of resident_factor.hpp.
 size_t resident_v_bytes(const Dims& d, size_t elem, int cls);
 size_t resident_l_bytes(const Dims& d, size_t elem, int cls);
