@@ -8,6 +8,16 @@ import torch
 TOL = {torch.float64: 1e-9, torch.float32: 1e-4, np.float64: 1e-9, np.float32: 1e-4}
 
 
+def on_path(solver, path):
+    """A TurboMPCSolver whose forward direct solve stays on the streaming kernel and its
+    stage records (path "streaming"), also where small batches run on-chip by default."""
+    from turbompc_amd import _lib
+
+    if path == "streaming":
+        solver._admm_solver_fwd._kernel_flags |= _lib.flag_stream_p(1)
+    return solver
+
+
 def rel_err(a, b) -> float:
     a = np.asarray(a.detach().cpu() if torch.is_tensor(a) else a, dtype=np.float64)
     b = np.asarray(b.detach().cpu() if torch.is_tensor(b) else b, dtype=np.float64)

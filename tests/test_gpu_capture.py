@@ -33,12 +33,17 @@ def _initial_state(qp, rho):
             torch.full((B,), float(rho), dtype=qp.dtype, device=DEV)]
 
 
+# INVARIANT_A alone keeps the streaming kernel and its form; with ANY_FORM the call runs on-chip
+FORMS = {"ainv": 0, "on-chip": _lib.FLAG_ANY_FORM}
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-def test_admm_direct_ainv_call_replays_in_a_graph(dtype):
+@pytest.mark.parametrize("form", list(FORMS))
+def test_admm_direct_ainv_call_replays_in_a_graph(dtype, form):
     prob = make_quadrotor_config(B=96, seed=5, dtype=dtype, device=DEV)
     qp = prob.build_qp(*prob.initial_guess())
     B, T, n, nx, n0, m = qp.dims
-    flags = _lib.FLAG_STD_DYNAMICS | _lib.FLAG_DIAG_COST | _lib.FLAG_CONST_G | _lib.FLAG_INVARIANT_A
+    flags = _lib.FLAG_STD_DYNAMICS | _lib.FLAG_DIAG_COST | _lib.FLAG_CONST_G | _lib.FLAG_INVARIANT_A | FORMS[form]
     cfg = cfg_struct(max_iter=20, check_every=10, adapt_rho_every=0, pcg_max_iter=0, use_slack=False, flags=flags,
                      sigma=1e-6, eps_abs=1e-30, eps_rel=1e-30, rho_min=1e-6, rho_max=1e6,
                      adaptive_rho_tolerance=5.0, rho_f_factor=1000.0, alpha=1.6, pcg_eps=0.0)
@@ -92,7 +97,8 @@ def test_admm_direct_ainv_call_replays_in_a_graph(dtype):
     del keep
 
 
-def test_admm_direct_ainv_calls_from_two_threads():
+@pytest.mark.parametrize("form", list(FORMS))
+def test_admm_direct_ainv_calls_from_two_threads(form):
     """Two host threads, each with its own stream and workspace, call the
     forking solve at the same time (each thread forks its own side stream):
     every call equals the same call made alone, bit for bit."""
@@ -101,7 +107,7 @@ def test_admm_direct_ainv_calls_from_two_threads():
     dtype = torch.float32
     probs = [make_quadrotor_config(B=64 + 32 * k, seed=7 + k, dtype=dtype, device=DEV) for k in range(2)]
     qps = [p.build_qp(*p.initial_guess()) for p in probs]
-    flags = _lib.FLAG_STD_DYNAMICS | _lib.FLAG_DIAG_COST | _lib.FLAG_CONST_G | _lib.FLAG_INVARIANT_A
+    flags = _lib.FLAG_STD_DYNAMICS | _lib.FLAG_DIAG_COST | _lib.FLAG_CONST_G | _lib.FLAG_INVARIANT_A | FORMS[form]
     cfg = cfg_struct(max_iter=20, check_every=10, adapt_rho_every=0, pcg_max_iter=0, use_slack=False, flags=flags,
                      sigma=1e-6, eps_abs=1e-30, eps_rel=1e-30, rho_min=1e-6, rho_max=1e6,
                      adaptive_rho_tolerance=5.0, rho_f_factor=1000.0, alpha=1.6, pcg_eps=0.0)

@@ -23,7 +23,7 @@ import pytest
 import torch
 
 import oracle
-from helpers import np_qp, random_qp, rel_err, zero_state
+from helpers import np_qp, on_path, random_qp, rel_err, zero_state
 from turbompc_amd import _lib
 from turbompc_amd.problems.quadrotor import make_quadrotor_config
 from turbompc_amd.solvers.admm.admm import ADMMSolver, ADMMState
@@ -211,8 +211,9 @@ def test_invariant_a_mask_read_back(kind):
 
 
 def test_quadrotor_sqp_invariant_a_default_and_bit_equal():
-    """The benchmark's SQP solve (quadrotor, fp32): the solver turns the form
-    on with the resident G rows, and the iterates equal those without it."""
+    """The benchmark's SQP solve (quadrotor, fp32): the solver offers the form
+    with the resident G rows, and on the streaming kernel (this batch runs
+    on-chip by default) the iterates equal those without it."""
     import copy
 
     from turbompc_amd.solvers.turbompc_solver import DEFAULT_SOLVER_PARAMS, TurboMPCSolver
@@ -225,10 +226,13 @@ def test_quadrotor_sqp_invariant_a_default_and_bit_equal():
     for inv in (True, False):
         solver = TurboMPCSolver(prob, params)
         assert solver._admm_solver_fwd._kernel_flags & _lib.FLAG_INVARIANT_A
+        default = solver.solve(solver.initial_guess())
+        on_path(solver, "streaming")
         if not inv:
             solver._admm_solver_fwd._kernel_flags &= ~_lib.FLAG_INVARIANT_A
         sols.append(solver.solve(solver.initial_guess()))
     torch.cuda.synchronize()
+    assert not torch.equal(default.states, sols[0].states)
     for k in ("states", "controls"):
         assert torch.equal(getattr(sols[0], k), getattr(sols[1], k)), k
     for k in sols[0].admm_state._fields:

@@ -8,7 +8,7 @@ import copy
 
 import pytest
 import torch
-from helpers import rel_err
+from helpers import on_path, rel_err
 
 from turbompc_amd.problems import configs
 from turbompc_amd.problems.quadrotor import make_quadrotor_config
@@ -180,14 +180,23 @@ def test_device_loop_equals_masked_with_a_nonfinite_problem(mode):
     _assert_same(dev, msk)
 
 
+def _assert_path(sol, prob, params, path):
+    """The streaming kernel's iterates are not the default's, bit for bit."""
+    if path == "streaming":
+        other = TurboMPCSolver(prob, params)
+        assert not torch.equal(other.solve(other.initial_guess()).states, sol.states)
+
+
+@pytest.mark.parametrize("path", ["default", "streaming"])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("stop", [False, True])
-def test_quadrotor_step_linearization_equals_build_qp(dtype, stop):
+def test_quadrotor_step_linearization_equals_build_qp(dtype, stop, path):
     """The quadrotor's SQP steps build their own dynamics rows
     (tmpc_sqp_admm_step_quadrotor_*: the linearization at the step's input
-    iterate, written into the QP buffers and straight into the stage
-    records): the solve is bit for bit the one whose loop builds each QP
-    with build_qp and lets the step copy the rows into the records."""
+    iterate, written into the QP buffers and, on the streaming kernel, straight
+    into the stage records): the solve is bit for bit the one whose loop builds
+    each QP with build_qp and lets the step copy the rows into the records.  By
+    default this batch runs on-chip, without records."""
     prob = make_quadrotor_config(B=24, seed=7, dtype=dtype, device="cuda")
     params = _params(6, 20, 0.0, linesearch=False, criterion="first_order")
     if stop:
@@ -198,9 +207,10 @@ def test_quadrotor_step_linearization_equals_build_qp(dtype, stop):
         if not fused:
             p.step_linearization = lambda: None  # noqa: E731  the build_qp path
         assert (p.step_linearization() is not None) == fused
-        solver = TurboMPCSolver(p, params)
+        solver = on_path(TurboMPCSolver(p, params), path)
         out.append(solver.solve(solver.initial_guess()))
     torch.cuda.synchronize()
+    _assert_path(out[0], prob, params, path)
     _assert_same(*out)
     if stop:
         assert len(set(out[0].num_iter.tolist())) >= 2
@@ -231,8 +241,9 @@ def _planar_obstacles(B, seed):
         obstacles_dimension=2)
 
 
+@pytest.mark.parametrize("path", ["default", "streaming"])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
-def test_obstacle_step_on_padded_records_equals_build_qp(dtype):
+def test_obstacle_step_on_padded_records_equals_build_qp(dtype, path):
     """The obstacle SQP step where the stage records are wider than the QP
     (n = 6 padded to 9): the step writes the obstacle rows into the QP only
     and the library copies G, l, u into the records; the solve equals the
@@ -244,17 +255,19 @@ def test_obstacle_step_on_padded_records_equals_build_qp(dtype):
         p = copy.copy(prob)
         if not fused:
             p.step_linearization = lambda: None  # noqa: E731  the build_qp path
-        solver = TurboMPCSolver(p, params)
+        solver = on_path(TurboMPCSolver(p, params), path)
         out.append(solver.solve(solver.initial_guess()))
     torch.cuda.synchronize()
+    _assert_path(out[0], prob, params, path)
     assert bool(torch.isfinite(out[0].states).all())
     _assert_same(*out)
 
 
+@pytest.mark.parametrize("path", ["default", "streaming"])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("stop", [False, True])
 @pytest.mark.parametrize("slack", [False, True])
-def test_obstacle_step_linearization_equals_build_qp(dtype, stop, slack):
+def test_obstacle_step_linearization_equals_build_qp(dtype, stop, slack, path):
     """Config 4's SQP steps build their own obstacle rows
     (tmpc_sqp_admm_step_obstacle_*: the linearization at the step's input
     iterate, written into the QP's G, l, u and straight into the stage
@@ -272,9 +285,10 @@ def test_obstacle_step_linearization_equals_build_qp(dtype, stop, slack):
         if not fused:
             p.step_linearization = lambda: None  # noqa: E731  the build_qp path
         assert (p.step_linearization() is not None) == fused
-        solver = TurboMPCSolver(p, params)
+        solver = on_path(TurboMPCSolver(p, params), path)
         out.append(solver.solve(solver.initial_guess()))
     torch.cuda.synchronize()
+    _assert_path(out[0], prob, params, path)
     _assert_same(*out)
     if stop:
         assert len(set(out[0].num_iter.tolist())) >= 2

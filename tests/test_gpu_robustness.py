@@ -76,13 +76,13 @@ def _poisoned(qp: QPData, b: int) -> QPData:
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("path", ["stream", "generic", "pcg"])
+@pytest.mark.parametrize("path", ["default", "stream", "generic", "pcg"])
 def test_nonfinite_flag_marks_exactly_the_poisoned_problem(dtype, path):
     B, T, n, nx, m = 7, 9, 6, 4, 2  # nx + m <= n: the streaming kernel's shape
     qp = random_qp(B, T, n, nx, m, seed=5, std=True, diag=True).to(DEV, dtype)
     bad = 4
     qp = _poisoned(qp, bad)
-    flags = _lib.FLAG_GENERIC_KERNEL if path == "generic" else 0
+    flags = {"generic": _lib.FLAG_GENERIC_KERNEL, "stream": _lib.flag_stream_p(1)}.get(path, 0)
     backend = AdmmBackend.HIP_PCG if path == "pcg" else AdmmBackend.HIP_DIRECT
     solver = ADMMSolver(ZShape(T - 1, nx, n - nx), {"max_iter": 20, "tol_epsilon": 1e-8}, sigma=1e-6, max_iter=12,
                         eps_abs=1e-30, eps_rel=1e-30, check_termination_every=5, adapt_rho_every=0,

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 import oracle
-from helpers import TOL, rel_err
+from helpers import TOL, on_path, rel_err
 from oracle.sqp_cpu import quadrotor_sqp
 from turbompc_amd.problems.quadrotor import make_quadrotor_config
 from turbompc_amd.solvers.turbompc_solver import DEFAULT_SOLVER_PARAMS, TurboMPCSolver
@@ -277,15 +277,18 @@ def test_sqp_step_check_and_activity(kernel, use_slack, dtype):
         np.testing.assert_array_equal(a[on], p[on])
 
 
+@pytest.mark.parametrize("path", ["default", "streaming"])
 @pytest.mark.parametrize("case", ["quadrotor", "config4", "config4-slack", "config4-built", "config4-built-slack"])
-def test_sqp_warm_records_match_repacking(case):
+def test_sqp_warm_records_match_repacking(case, path):
     """FLAG_WARM_RECORDS: an SQP solve whose steps rewrite only the records
     that changed gives the same iterates, bit for bit, as one that repacks
     every record at every step.  The quadrotor's and config 4's steps write
     their relinearized rows (A_minus and c; the obstacle rows of G, l, u) into
     the records themselves and keep the rest (config 4's dynamics records with
     FLAG_WARM_SAME_DYNAMICS); "built": config 4 with each QP from build_qp,
-    whose obstacle rows the step copies in (FLAG_WARM_INEQ)."""
+    whose obstacle rows the step copies in (FLAG_WARM_INEQ).  By default this
+    batch runs on-chip, where there are no records to keep: the flag changes
+    nothing."""
     import turbompc_amd.solvers.turbompc_solver as ts
     from turbompc_amd.problems import configs
 
@@ -300,7 +303,7 @@ def test_sqp_warm_records_match_repacking(case):
         if "built" in case:
             prob.step_linearization = lambda: None  # noqa: E731
             level = "constraints"
-    solver = TurboMPCSolver(prob, _params(n_sqp, iters))
+    solver = on_path(TurboMPCSolver(prob, _params(n_sqp, iters)), path)
     seen = []
     orig = ts._warm_level
     try:
@@ -312,6 +315,9 @@ def test_sqp_warm_records_match_repacking(case):
         ts._warm_level = orig
     torch.cuda.synchronize()
     assert seen and all(v == level for v in seen), seen
+    if path == "streaming":  # not the default's kernel
+        other = TurboMPCSolver(prob, _params(n_sqp, iters))
+        assert not torch.equal(other.solve(other.initial_guess()).states, warm.states)
     assert torch.equal(warm.states, cold.states) and torch.equal(warm.controls, cold.controls)
     assert torch.equal(warm.admm_state.y_f_dyn, cold.admm_state.y_f_dyn)
     assert torch.equal(warm.admm_state.y_g, cold.admm_state.y_g)

@@ -85,13 +85,13 @@ def test_config2_pcg_tolerance_stopped_at_100_iterations(kernel, dtype):
         assert e < bar, (k, e, bar)
 
 
-@pytest.mark.parametrize("kernel", ["stream", "generic"])
+@pytest.mark.parametrize("kernel", ["default", "stream", "generic"])
 def test_config5_fixed_rho_at_200_iterations_fp64(kernel):
     prob = configs.config5(B=64, seed=0)
     qp = prob.build_qp(*prob.initial_guess())
     cfg = oracle.OracleCfg(max_iter=200, check_every=25, adapt_rho_every=0, sigma=1e-6, eps_abs=1e-9,
                            eps_rel=1e-9, rho_f_factor=1000.0, alpha=1.6)
-    flags = _lib.FLAG_GENERIC_KERNEL if kernel == "generic" else 0
+    flags = {"generic": _lib.FLAG_GENERIC_KERNEL, "stream": _lib.flag_stream_p(1)}.get(kernel, 0)
     print(f"config 5 ({kernel}): 200 ADMM iterations, fixed rho, B=64, fp64", flush=True)
     ref, it_ref, _, out, stats = _run_pair(qp, cfg, torch.float64, kernel_flags=flags, diag_cost=True)
     np.testing.assert_array_equal(stats.num_iter.cpu().numpy(), it_ref)
