@@ -50,7 +50,7 @@ VALU_PEAK_TFLOPS = 78.6
 
 def bytes_per_qp(T, n, nx, n0, m, K, w, m_g=0):
     """Algorithmic HBM bytes of one QP solve: w * (F + K * I), the streaming
-    model of the survey (factor written once and read once per iteration;
+    model (factor written once and read once per iteration;
     QP data and iterates read/written once per iteration; A_plus, A0 and
     box-selector G rows are constants and not counted)."""
     N = T - 1
@@ -75,6 +75,26 @@ def bytes_pcg(T, n, nx, n0, m, K, pcg_iters, w, m_g=0):
     per_pcg = sp + 9 * T * n
     phase = K * It + pcg_iters * per_pcg
     return w * (F + phase), w * phase
+
+
+def flops_admm_on_chip(T, n, nx, m):
+    """Algorithmic flops of one ADMM iteration of the on-chip kernel per problem
+    (csrc/resident.hpp), 2 per multiply-add and stage: the two passes over the
+    states and Theta^-1 r between them (nx x nx each), the controls (A_u^T x,
+    Suu^-1, Kx), the products with [A; G] and their transposes, Kx^T and Kn^T."""
+    nu = n - nx
+    return 2 * T * (3 * nx * nx + 2 * nx * nu + nu * nu + 2 * (nx + m) * n + 2 * nx * nu)
+
+
+def bytes_admm_on_chip(T, n, nx, n0, m, w):
+    """What one launch of the on-chip kernel moves per problem: the factor (V in
+    rows of whole 16-byte chunks, L), A, A0, G and the vectors of the QP in, the
+    state in and out.  The blocks then stay in LDS and registers."""
+    nu, lanes = n - nx, 16 // w
+    factor = T * (-(-nx // lanes) * lanes * nx + (nx + 2 * nu) * n)
+    qp = (T - 1) * nx * (n + 1) + n0 * (n + 1) + m * n + T * (n + 2 * m)
+    state = T * (n + 2 * m) + n0 + (T - 1) * nx
+    return w * (factor + qp + 2 * state)
 
 
 def flops_pcg_iteration(T, n):
@@ -454,9 +474,11 @@ def run_config5(args, dev):
     bwd_avg_ms = sum(bwd) / len(bwd)
     copy_calibration(args, dev)
     T = prob.horizon + 1
-    per_qp, F, It = bytes_per_qp(T, 9, 6, 6, 3, K, 8)
-    iter_bytes = B * K * It
-    achieved = iter_bytes / iter_avg_s / 1e9
+    # the blocks stay in LDS and registers over a launch, so the kernel is not bound by
+    # HBM: its roofline is the algorithmic flop rate against the fp64 VALU peak
+    flops = B * K * flops_admm_on_chip(T, 9, 6, 3)
+    moved = B * bytes_admm_on_chip(T, 9, 6, 6, 3, 8)
+    tflops, gbs = flops / iter_avg_s / 1e12, moved / iter_avg_s / 1e9
     finite = bool(all(torch.isfinite(g).all() for g in grads) and torch.isfinite(sol.states).all())
     line = base_line(f"MPC solves/sec at B={B}, config 5 forward + gradient (1 MI355X)", B * args.steps / elapsed,
                      args, elapsed, "f64",
@@ -469,13 +491,16 @@ def run_config5(args, dev):
                          "batch": B, "horizon": prob.horizon, "admm_iterations": K,
                          "parallelism": "single GPU, batch-parallel", "solution_finite": finite,
                          "forward_qp_solve_ms": solve_avg_s * 1e3, "backward_ms": bwd_avg_ms})
-    line["roofline"] = roofline(
-        achieved, None, f"admm_resident_kernel, fp64 (one launch = {K} ADMM iterations of the batch; the bytes are the "
-        "streaming model's, which this kernel does not move: its blocks stay in LDS and registers)", iter_bytes,
-        iter_avg_s * 1e3,
-        qp_solve={"kernels": "resident_factor + admm_resident", "algorithmic_bytes": per_qp * B,
-                  "avg_ms": solve_avg_s * 1e3, "achieved": per_qp * B / solve_avg_s / 1e9,
-                  "frac": per_qp * B / solve_avg_s / 1e9 / HBM_PEAK_GBS})
+    line["roofline"] = {
+        "bound": "valu", "achieved": tflops, "peak": VALU_PEAK_TFLOPS, "unit": "TFLOP/s",
+        "frac": tflops / VALU_PEAK_TFLOPS, "traffic": None,
+        "kernel": f"admm_resident_kernel, fp64 (one launch = {K} ADMM iterations of the batch)",
+        "algorithmic_flops_per_launch": flops, "avg_launch_ms": iter_avg_s * 1e3,
+        "note": "two serial passes over the states (T / 2 steps each, by one wavefront of a problem's workgroup) take "
+                "most of an iteration",
+        "hbm": {"bytes_per_launch": moved, "achieved": gbs, "frac": gbs / HBM_PEAK_GBS,
+                "note": "factor, QP and state once per launch"},
+        "qp_solve": {"kernels": "resident_factor + admm_resident", "avg_ms": solve_avg_s * 1e3}}
     return line
 
 

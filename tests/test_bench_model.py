@@ -55,3 +55,13 @@ def test_pcg_flop_model():
     # (3T - 2) n^2 entries, 2 flop each, for both products; 2 dots + 3 updates
     T, n = 51, 16
     assert bench.flops_pcg_iteration(T, n) == 2 * 2 * (3 * T - 2) * n * n + (2 * 2 + 3 * 2) * T * n
+
+
+def test_on_chip_admm_model():
+    # one stage of nx = 6, n = 9, m = 3 (nu = 3): 3 x 36 state products, 18 + 18 control
+    # couplings each way, 9, and 9 rows of 9 entries twice: 351 multiply-adds
+    T = 101
+    assert bench.flops_admm_on_chip(T, 9, 6, 3) == 2 * T * (3 * 36 + 2 * 18 + 9 + 2 * 81 + 2 * 18)
+    # V rows of 6 fp64 words (three 16-byte chunks), L of (6 + 6) x 9
+    words = T * (36 + 108) + (T - 1) * 60 + 60 + 27 + T * 15 + 2 * (T * 15 + 6 + (T - 1) * 6)
+    assert bench.bytes_admm_on_chip(T, 9, 6, 6, 3, 8) == 8 * words
