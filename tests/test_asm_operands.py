@@ -27,6 +27,11 @@ __global__ void source_fma(const R* p, R* o) {
   o[threadIdx.x] = row_fma<0>(row<R, N>(p).w, g, g);
 }
 template <typename R, int N>
+__global__ void source_sum(const R* p, R* o) {
+  const R g = p[threadIdx.x];
+  o[threadIdx.x] = row_fma_sum(row<R, N>(p).w, g, g, p[threadIdx.x + 8192]);
+}
+template <typename R, int N>
 __global__ void source_x2(const R* p, R* o) {
   R g = p[threadIdx.x], a = g, b = R(1);
   row_fma_x2<0>(g, row<R, N>(p).w, a, row<R, N>(p + 4096).w, b);
@@ -69,6 +74,8 @@ __global__ void source_dot(const double* p, double* o) {
 template __global__ void source_fma<float, 4>(const float*, float*);
 template __global__ void source_fma<float, 13>(const float*, float*);
 template __global__ void source_fma<double, 6>(const double*, double*);
+template __global__ void source_sum<float, 13>(const float*, float*);
+template __global__ void source_sum<double, 6>(const double*, double*);
 template __global__ void source_x2<float, 3>(const float*, float*);
 template __global__ void source_x2<double, 4>(const double*, double*);
 template __global__ void source_2<float, 12>(const float*, float*);
@@ -97,9 +104,9 @@ def test_accumulators_share_no_register_with_a_later_source(assembly):
             kernel = block[0]
             continue
         written = set()
-        for op in re.findall(r"v_(?:fmac|mul)_f(?:32|64)_dpp (\S+), (\S+), (\S+) row_newbcast", block[1]):
+        for op in re.findall(r"v_(?:fmac|mul|add)_f(?:32|64)(?:_dpp)? ([^\s,]+), ([^\s,]+), ([^\s,]+)", block[1]):
             bad += [(kernel, op)] if written & set(op[1:]) or op[0] in op[1:] else []
             written.add(op[0])
         blocks += bool(written)
-    assert blocks >= 12
+    assert blocks >= 14
     assert not bad, bad

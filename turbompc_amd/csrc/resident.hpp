@@ -16,13 +16,13 @@
 //   C2  x_t = w_t + V_t^T x (outwards)
 //   P2  u_t = Suu^-1 (gu_t + rho_f A_u^T x_{t+1}) - Kx x_t, products, relaxation,
 //       projection, duals, gamma_t -> gx_t = gamma_x - Kx^T gu, h_t  (all stages)
-// with a workgroup barrier after each.  Cycles of an iteration (C1, P1, C2, P2, waits
-// and the rest): fp32, T = 41, NX = 13, alone on its CU 3380 + 1140 + 3750 + 4360 +
-// 3150, two workgroups on each 4340 + 2000 + 4120 + 9170 + 3130; fp64, T = 101,
-// NX = 6 5730 + 1770 + 7330 + 7480 + 1940.  QP solves of 20 iterations against the
-// streaming kernel, which reads every record twice per iteration and walks all T
-// stages in turn, are listed at the shape classes (resident.hip): 1412 -> 319 us for
-// 256 problems of T = 41, NX = 13 in fp32.
+// with a workgroup barrier after each.  Cycles of an iteration seen by wavefront 0 (C1,
+// P1, C2, P2, barriers and the rest): fp32, T = 41, NX = 13, alone on its CU 4190 + 960 +
+// 3990 + 4500 + 1780, two workgroups on each 4610 + 2000 + 3730 + 8490 + 2410; fp64, T =
+// 101, NX = 6 6810 + 1430 + 6170 + 8480 + 1530.  QP solves against the streaming kernel,
+// which reads every record twice per iteration and walks all T stages in turn, are listed
+// at the shape classes (resident.hip): 1412 -> 319 us for 20 iterations of 256 problems of
+// T = 41, NX = 13 in fp32.
 //
 // A stage is a group of GL lanes: GL = 32 has the states (and dynamics rows) in the
 // first 16-lane row, the controls at lanes 16 .. 16 + NU - 1 and the inequality
@@ -551,8 +551,14 @@ __global__ __launch_bounds__(TPB, WPE) void admm_resident_kernel(ResArgs<R> a) {
         ld_row(c[(k + CB - 1) % CB], q + (k + CB - 1) * CW);
         q[k * CW + CX + lr] = r;
         // (gx and h first: each alone is as large as the duals, and would be rounded so with
-        // every term: fp32, T = 51, NX = 12 states 1.29e-6 off 64 bits, 7.1e-7 like this)
-        r = row_fma<0>(c[k].w, r, c[(k + 1) % CB].g + c[(k + 1) % CB].h);
+        // every term: fp32, T = 51, NX = 12 states 1.29e-6 off 64 bits, 7.1e-7 like this.
+        // With two sets they were fetched in this step, and the wait for them is better
+        // not tied to the chain's first instruction: fp64, NX = 13 5080 cycles against 5703)
+        const CBuf& e = c[(k + 1) % CB];
+        if constexpr (CB > 2)
+          r = row_fma_sum(c[k].w, r, e.g, e.h);
+        else
+          r = row_fma<0>(c[k].w, r, e.g + e.h);
       };
       int p = mid;
       for (; p > CB; p -= CB, q += CB * CW) {

@@ -229,6 +229,161 @@ __device__ __forceinline__ double row_fma(const double (&w)[13], double s, doubl
   return acc + odd;
 }
 
+// (g + h) + sum_k w[k] s(lane k), k < N.  The sum of g and h is formed in the block, in the
+// place of a wait state: formed before it, the compiler waits for g and h ahead of the
+// loads that the caller has in flight (a chain of fp64, T = 101, NX = 6 7270 cycles, 6810
+// like this).
+
+__device__ __forceinline__ float row_fma_sum(const float (&w)[4], float s, float g, float h) {
+  float acc, odd;
+  asm volatile(
+      "s_nop 0\n"
+      "v_add_f32 %0, %3, %4\n"
+      "v_fmac_f32_dpp %0, %2, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+      "v_mul_f32_dpp %1, %2, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf"
+      : "=&v"(acc), "=&v"(odd)
+      : "v"(s), "v"(g), "v"(h), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]));
+  return acc + odd;
+}
+
+__device__ __forceinline__ float row_fma_sum(const float (&w)[6], float s, float g, float h) {
+  float acc, odd;
+  asm volatile(
+      "s_nop 0\n"
+      "v_add_f32 %0, %3, %4\n"
+      "v_fmac_f32_dpp %0, %2, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+      "v_mul_f32_dpp %1, %2, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf"
+      : "=&v"(acc), "=&v"(odd)
+      : "v"(s), "v"(g), "v"(h), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]));
+  return acc + odd;
+}
+
+__device__ __forceinline__ float row_fma_sum(const float (&w)[12], float s, float g, float h) {
+  float acc, odd;
+  asm volatile(
+      "s_nop 0\n"
+      "v_add_f32 %0, %3, %4\n"
+      "v_fmac_f32_dpp %0, %2, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+      "v_mul_f32_dpp %1, %2, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %11 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %12 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %13 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %14 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %15 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %16 row_newbcast:11 row_mask:0xf bank_mask:0xf"
+      : "=&v"(acc), "=&v"(odd)
+      : "v"(s), "v"(g), "v"(h), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]));
+  return acc + odd;
+}
+
+__device__ __forceinline__ float row_fma_sum(const float (&w)[13], float s, float g, float h) {
+  float acc, odd;
+  asm volatile(
+      "s_nop 0\n"
+      "v_add_f32 %0, %3, %4\n"
+      "v_fmac_f32_dpp %0, %2, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+      "v_mul_f32_dpp %1, %2, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %11 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %12 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %13 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %14 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %15 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %1, %2, %16 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f32_dpp %0, %2, %17 row_newbcast:12 row_mask:0xf bank_mask:0xf"
+      : "=&v"(acc), "=&v"(odd)
+      : "v"(s), "v"(g), "v"(h), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]));
+  return acc + odd;
+}
+
+__device__ __forceinline__ double row_fma_sum(const double (&w)[4], double s, double g, double h) {
+  double acc, odd = 0.0;
+  asm volatile(
+      "s_nop 0\n"
+      "v_add_f64 %0, %3, %4\n"
+      "v_fmac_f64_dpp %0, %2, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf"
+      : "=&v"(acc), "+&v"(odd)
+      : "v"(s), "v"(g), "v"(h), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]));
+  return acc + odd;
+}
+
+__device__ __forceinline__ double row_fma_sum(const double (&w)[6], double s, double g, double h) {
+  double acc, odd = 0.0;
+  asm volatile(
+      "s_nop 0\n"
+      "v_add_f64 %0, %3, %4\n"
+      "v_fmac_f64_dpp %0, %2, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf"
+      : "=&v"(acc), "+&v"(odd)
+      : "v"(s), "v"(g), "v"(h), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]));
+  return acc + odd;
+}
+
+__device__ __forceinline__ double row_fma_sum(const double (&w)[12], double s, double g, double h) {
+  double acc, odd = 0.0;
+  asm volatile(
+      "s_nop 0\n"
+      "v_add_f64 %0, %3, %4\n"
+      "v_fmac_f64_dpp %0, %2, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %11 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %12 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %13 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %14 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %15 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %16 row_newbcast:11 row_mask:0xf bank_mask:0xf"
+      : "=&v"(acc), "+&v"(odd)
+      : "v"(s), "v"(g), "v"(h), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]));
+  return acc + odd;
+}
+
+__device__ __forceinline__ double row_fma_sum(const double (&w)[13], double s, double g, double h) {
+  double acc, odd = 0.0;
+  asm volatile(
+      "s_nop 0\n"
+      "v_add_f64 %0, %3, %4\n"
+      "v_fmac_f64_dpp %0, %2, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %11 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %12 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %13 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %14 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %15 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %1, %2, %16 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
+      "v_fmac_f64_dpp %0, %2, %17 row_newbcast:12 row_mask:0xf bank_mask:0xf"
+      : "=&v"(acc), "+&v"(odd)
+      : "v"(s), "v"(g), "v"(h), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "v"(w[4]), "v"(w[5]), "v"(w[6]), "v"(w[7]), "v"(w[8]), "v"(w[9]), "v"(w[10]), "v"(w[11]), "v"(w[12]));
+  return acc + odd;
+}
+
 // Two or three such sums side by side, one chain each (in place): independent
 // chains leave no stall between dependent instructions (one chain alone issues every
 // 8.4 cycles, two every 6.5, three and more every 5.1).
