@@ -86,13 +86,14 @@ def flops_admm_on_chip(T, n, nx, m):
     return 2 * T * (3 * nx * nx + 2 * nx * nu + nu * nu + 2 * (nx + m) * n + 2 * nx * nu)
 
 
-def bytes_admm_on_chip(T, n, nx, n0, m, w):
+def bytes_admm_on_chip(T, n, nx, n0, m, w, const_g=True):
     """What one launch of the on-chip kernel moves per problem: the factor (V in
-    rows of whole 16-byte chunks, L), A, A0, G and the vectors of the QP in, the
-    state in and out.  The blocks then stay in LDS and registers."""
+    rows of whole 16-byte chunks, L), A, A0, G (one, or one per stage) and the
+    vectors of the QP in, the state in and out.  The blocks then stay in LDS and
+    registers."""
     nu, lanes = n - nx, 16 // w
     factor = T * (-(-nx // lanes) * lanes * nx + (nx + 2 * nu) * n)
-    qp = (T - 1) * nx * (n + 1) + n0 * (n + 1) + m * n + T * (n + 2 * m)
+    qp = (T - 1) * nx * (n + 1) + n0 * (n + 1) + (1 if const_g else T) * m * n + T * (n + 2 * m)
     state = T * (n + 2 * m) + n0 + (T - 1) * nx
     return w * (factor + qp + 2 * state)
 
@@ -375,6 +376,30 @@ def roofline(achieved, traffic, kernel, bytes_per_launch, avg_ms, **extra):
     return r
 
 
+def roofline_on_chip(B, K, T, n, nx, n0, m, w, const_g, solve_avg_s, iter_avg_s):
+    """The on-chip kernel's blocks stay in LDS and registers over a launch, so HBM does
+    not bound it: its algorithmic flop rate against the VALU peak, and beside it the
+    bytes a launch moves."""
+    flops = B * K * flops_admm_on_chip(T, n, nx, m)
+    moved = B * bytes_admm_on_chip(T, n, nx, n0, m, w, const_g)
+    tflops, gbs = flops / iter_avg_s / 1e12, moved / iter_avg_s / 1e9
+    return {"bound": "valu", "achieved": tflops, "peak": VALU_PEAK_TFLOPS, "unit": "TFLOP/s",
+            "frac": tflops / VALU_PEAK_TFLOPS, "traffic": None,
+            "kernel": f"admm_resident_kernel (one launch = {K} ADMM iterations of the batch)",
+            "algorithmic_flops_per_launch": flops, "avg_launch_ms": iter_avg_s * 1e3,
+            "note": "two serial passes over the states (T / 2 steps each, by one wavefront of a problem's workgroup) "
+                    "take 0.4 to 0.55 of an iteration",
+            "hbm": {"bytes_per_launch": moved, "achieved": gbs, "frac": gbs / HBM_PEAK_GBS,
+                    "note": "factor, QP and state once per launch"},
+            "qp_solve": {"kernels": "resident_factor + admm_resident", "avg_ms": solve_avg_s * 1e3}}
+
+
+def runs_on_chip(c4, B, iters):
+    """Whether config 3's or 4's QPs of B problems run on the on-chip path (the
+    library's rule for these shapes, csrc/resident.hip)."""
+    return B <= (2048 if c4 or iters < 5 else 3072)
+
+
 # --------------------------------------------------------------- workloads ----
 def run_sqp_workload(args, dev):
     """config3 (the metric) and config4: the SQP solve from the same guess."""
@@ -420,6 +445,10 @@ def run_sqp_workload(args, dev):
                          "workload": workload, "batch": B, "horizon": prob.horizon, "sqp_iterations": args.sqp,
                          "admm_iterations": args.admm_iters, "parallelism": "single GPU, batch-parallel",
                          "solution_finite": finite, "kernel_only_solves_per_s": B / (args.sqp * solve_avg_s)})
+    if runs_on_chip(c4, B, args.admm_iters):
+        dims = (T, 9, 6, 6, 11, 4, False) if c4 else (T, 17, 13, 13, 4, 4, True)
+        line["roofline"] = roofline_on_chip(B, args.admm_iters, *dims, solve_avg_s, iter_avg_s)
+        return line
     line["roofline"] = roofline(
         achieved, None if c4 else measured_traffic(B, args.admm_iters),
         f"admm_stream_kernel (one launch = {args.admm_iters} ADMM iterations of the batch)", iter_bytes,
@@ -474,11 +503,6 @@ def run_config5(args, dev):
     bwd_avg_ms = sum(bwd) / len(bwd)
     copy_calibration(args, dev)
     T = prob.horizon + 1
-    # the blocks stay in LDS and registers over a launch, so the kernel is not bound by
-    # HBM: its roofline is the algorithmic flop rate against the fp64 VALU peak
-    flops = B * K * flops_admm_on_chip(T, 9, 6, 3)
-    moved = B * bytes_admm_on_chip(T, 9, 6, 6, 3, 8)
-    tflops, gbs = flops / iter_avg_s / 1e12, moved / iter_avg_s / 1e9
     finite = bool(all(torch.isfinite(g).all() for g in grads) and torch.isfinite(sol.states).all())
     line = base_line(f"MPC solves/sec at B={B}, config 5 forward + gradient (1 MI355X)", B * args.steps / elapsed,
                      args, elapsed, "f64",
@@ -491,16 +515,7 @@ def run_config5(args, dev):
                          "batch": B, "horizon": prob.horizon, "admm_iterations": K,
                          "parallelism": "single GPU, batch-parallel", "solution_finite": finite,
                          "forward_qp_solve_ms": solve_avg_s * 1e3, "backward_ms": bwd_avg_ms})
-    line["roofline"] = {
-        "bound": "valu", "achieved": tflops, "peak": VALU_PEAK_TFLOPS, "unit": "TFLOP/s",
-        "frac": tflops / VALU_PEAK_TFLOPS, "traffic": None,
-        "kernel": f"admm_resident_kernel, fp64 (one launch = {K} ADMM iterations of the batch)",
-        "algorithmic_flops_per_launch": flops, "avg_launch_ms": iter_avg_s * 1e3,
-        "note": "two serial passes over the states (T / 2 steps each, by one wavefront of a problem's workgroup) take "
-                "most of an iteration",
-        "hbm": {"bytes_per_launch": moved, "achieved": gbs, "frac": gbs / HBM_PEAK_GBS,
-                "note": "factor, QP and state once per launch"},
-        "qp_solve": {"kernels": "resident_factor + admm_resident", "avg_ms": solve_avg_s * 1e3}}
+    line["roofline"] = roofline_on_chip(B, K, T, 9, 6, 6, 3, 8, True, solve_avg_s, iter_avg_s)
     return line
 
 

@@ -76,9 +76,10 @@ typedef struct tmpc_state {
  * With TMPC_FLAG_DIAG_COST as well, small blocks (nx <= 13, n - nx <= 4, with
  * m <= 4 rows, m <= 12 for nx <= 6 and n - nx <= 3, m <= 16 for nx <= 12) and
  * horizons whose blocks fit a workgroup's LDS and registers run on-chip instead, one
- * problem per workgroup without stage records, for batches where that is the
- * faster path; the generic-kernel, bits 8-9 and TMPC_FLAG_FACTOR_GROUPS flags
- * keep the other kernels. */
+ * problem per workgroup without stage records, for batches and iteration counts
+ * where that is the faster path; the generic-kernel, bits 8-9 and
+ * TMPC_FLAG_FACTOR_GROUPS flags and TMPC_FLAG_INVARIANT_A without
+ * TMPC_FLAG_ANY_FORM keep the other kernels. */
 #define TMPC_FLAG_GENERIC_KERNEL 2u
 #define TMPC_FLAG_STREAM_P(p) (((uint32_t)(p) & 3u) << 8)
 /* tmpc_admm_pcg_* with TMPC_FLAG_STD_DYNAMICS runs the whole solve in one
@@ -125,7 +126,8 @@ typedef struct tmpc_state {
  * records then keeps the G rows of its stage blocks in LDS and streams only
  * the A_minus rows of the stage records in its backward sweep, as in its
  * forward sweep (fewer bytes per iteration; the same products, so the same
- * iterates bit for bit).  Ignored by the other paths and shapes. */
+ * iterates bit for bit).  The on-chip path keeps one G in LDS, which lets it take
+ * longer horizons.  Ignored by the other paths and shapes. */
 #define TMPC_FLAG_CONST_G 32u
 /* With TMPC_FLAG_CONST_G on the same n = 17 records (nx n <= 224, at most two
  * problems per wavefront, a workspace of the size
@@ -134,11 +136,12 @@ typedef struct tmpc_state {
  * device on every call; a rigid body's position and velocity columns, for
  * example) stay in LDS, and both sweeps stream only the others (the same
  * products, so the same iterates bit for bit).  Needs no promise from the
- * caller; ignored by the other paths and shapes. */
+ * caller.  Without TMPC_FLAG_ANY_FORM it asks for this form: the call stays off
+ * the on-chip path, which has no use for it and is the faster one for small
+ * batches.  Ignored by the other paths and shapes. */
 #define TMPC_FLAG_INVARIANT_A 64u
-/* TMPC_FLAG_INVARIANT_A is an offer and not a request: the direct solve may run
- * on the on-chip path, which has no use for it.  A call with that flag alone
- * keeps the streaming kernel's form. */
+/* With TMPC_FLAG_INVARIANT_A: that form is an offer for where the streaming
+ * kernel runs, and the call may run on-chip. */
 #define TMPC_FLAG_ANY_FORM (1u << 14)
 
 typedef struct tmpc_admm_cfg {

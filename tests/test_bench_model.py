@@ -65,3 +65,7 @@ def test_on_chip_admm_model():
     # V rows of 6 fp64 words (three 16-byte chunks), L of (6 + 6) x 9
     words = T * (36 + 108) + (T - 1) * 60 + 60 + 27 + T * 15 + 2 * (T * 15 + 6 + (T - 1) * 6)
     assert bench.bytes_admm_on_chip(T, 9, 6, 6, 3, 8) == 8 * words
+    assert bench.bytes_admm_on_chip(T, 9, 6, 6, 3, 8, const_g=False) == 8 * (words + (T - 1) * 27)
+    # the benchmark's batches stream; its small ones run on-chip
+    assert not bench.runs_on_chip(False, 4096, 20) and not bench.runs_on_chip(True, 16384, 30)
+    assert bench.runs_on_chip(False, 512, 20) and bench.runs_on_chip(True, 512, 30)

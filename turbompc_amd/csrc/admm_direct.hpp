@@ -471,7 +471,7 @@ __global__ __launch_bounds__(kWave) void admm_chunk_kernel(AdmmArgs<R> a) {
 
 // Schur-only exact solve S x = rhs from the factor of S (phi read from S).  The chain
 // over the stages bounds it: with PF (NC > 0) the rows of the next stage's blocks and
-// its vector entry are in flight while a stage is solved. 
+// its vector entry are in flight while a stage is solved.
 // T = 51, fp64, without / with PF: n = 16, 512 problems 111 / 70 us, 4096 (1024
 // wavefronts, where the reads bound it) 259 / 283; n = 17, 512 problems 136 / 72.
 template <typename R, int NC, bool PF = false>
