@@ -45,10 +45,10 @@ __host__ __device__ __forceinline__ constexpr int packed_size(int n) { return (n
 __host__ __device__ __forceinline__ constexpr int th_pitch(int n) { return (packed_size(n) + 3) & ~3; }
 
 // What a workspace of the direct solve holds between calls: word kRecordsWord is
-// kRecordsHeld after a streaming call (whose stage records a warm call keeps) and
-// something else after any other.  The streaming and generic paths have the factor
-// there, which no later call reads (a NaN of this payload is no value of theirs), the
-// on-chip path a control word of its own that it clears.
+// kRecordsHeld after a streaming call, whose stage records a warm call keeps.  There the
+// streaming and generic paths have the factor, which no later call reads (a NaN of this
+// payload is no value of theirs), and the on-chip path, which overwrites the records, a
+// control word of its own that it clears.
 constexpr int kRecordsWord = 3;
 constexpr uint32_t kRecordsHeld = 0xfff9c0deu;
 

@@ -104,7 +104,7 @@ struct C4 : Cls<13, 4, 4, 32, 4, 6, 6> {
   static constexpr int few(bool f64, int, bool chunked) { return f64 || chunked ? 8 : 5; }
   static constexpr bool takes(int B, bool f64, int k, int, Chunks c) {
     if (!f64) return per_cu_at_most(B, c != Chunks::kLong ? 8 : (k < 2 ? 10 : 12));
-    return within_rounds(B, c == Chunks::kTiny ? 0 : (c == Chunks::kShort || k < 2 ? 7 : 8));
+    return per_cu_at_most(B, 16) && within_rounds(B, c == Chunks::kTiny ? 0 : (c == Chunks::kShort || k < 2 ? 7 : 8));
   }
 };
 constexpr int kClasses = 5;
