@@ -31,8 +31,9 @@ constexpr size_t kLdsBytes = 160 * 1024;
 //     10038); of one iteration 0.80 at 2048, 1.10 at 3072; T = 42 (k = 1) 0.96 at 2560,
 //     1.06 at 3072
 //   C4 fp64, 3 SQP steps: T = 21 (k = 2) 0.86 at 2048, 0.89 at 4096, of 5 iterations 0.91
-//     and 0.99, of one 0.96 and 1.10; T = 25 (k = 1) 0.60 at 1792, 1.05 at 2048, 0.75 at
-//     3072, 1.10 at 4096; a chunk per iteration 0.73 at 1536, 1.12 at 2048, 1.14 at 3072
+//     and 0.99, of one 0.96 and 1.10; T = 25 (k = 1) 0.60 at 1792, 1.05 at 2048, 1.10 at
+//     4096, T = 36 0.72 at 2412, 0.85 at 3229; a chunk per iteration T = 21 0.73 at 1536,
+//     1.12 at 2048, T = 41 1.14 at 3072
 //   C1 fp32: T = 65 (k = 1) 0.84 at 3072, 1.07 at 4096; T = 57 (k = 2) 0.67 at 4096
 //   C1 fp64: T = 57 (k = 1) 0.95 at 4096, 1.01 at 16384, but in chunks of 25 (of 100) 1.05
 //     and 1.11, of 5 0.90 at 2048, 1.13 at 3072; T = 85, chunks of 25 0.64 and 0.84 (past
